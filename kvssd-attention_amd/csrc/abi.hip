@@ -120,10 +120,10 @@ int units_of_desc(const kvssd_decode_desc* d, int* units) {
 int plan_checked(const kvssd_decode_desc* desc, int units, const void* workspace, size_t workspace_bytes, int* kernel,
                  int* splits) {
   if (int rc = choose_kernel(*desc, kernel)) return rc;
-  *splits = plan_splits(*desc, units).splits;
-  const size_t need = split_partial_bytes(*splits, desc->query_heads, desc->head_dim);
+  const size_t need = split_partial_bytes(plan_splits(*desc, units).splits, desc->query_heads, desc->head_dim);
   if (workspace == nullptr || workspace_bytes < need)
     return arg_error("workspace too small: need " + std::to_string(need) + " bytes");
+  *splits = launch_splits(*desc, units).splits;
   return 0;
 }
 
@@ -189,7 +189,7 @@ int decode_call(const kvssd_decode_desc* desc, const void* query, const uint8_t*
   a.units = units;
   a.stream = static_cast<hipStream_t>(stream);
   SplitPartials parts = carve_partials(workspace, splits, desc->query_heads, desc->head_dim);
-  const SplitPlan plan = plan_splits(*desc, units);
+  const SplitPlan plan = launch_splits(*desc, units);
   if (kernel == KVSSD_KERNEL_STAGED && !staged_aligned(a)) {
     if (desc->kernel == KVSSD_KERNEL_STAGED)
       return arg_error("staged matrix-core kernel needs 16-byte aligned packed arrays and scales");

@@ -30,7 +30,7 @@ TIMELINE_OUT = PKG / "libkvssd_hip_timeline.so"
 FASTCALL_SRC = HERE / "fastcall.c"
 FASTCALL_OUT = PKG / ("_fastcall" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
 BUILD = HERE / "_build"
-SOURCES = ["abi.hip", "decode_general.hip", "decode_mfma.hip", "decode_staged.hip", "merge.hip", "codec.hip", "records.hip", "vllm_codec.hip"]
+SOURCES = ["abi.hip", "decode_general.hip", "decode_tile.hip", "decode_mfma.hip", "decode_staged.hip", "merge.hip", "codec.hip", "records.hip", "vllm_codec.hip"]
 ARCH = "gfx950"
 
 COMMON = [

@@ -52,10 +52,20 @@ struct SplitPlan {
   int splits;            // partitions of the attended blocks
   int blocks_per_split;  // consecutive attended blocks per partition
 };
+// the most splits a shape's partials take (the workspace size)
 SplitPlan plan_splits(const kvssd_decode_desc& d, int units);
+// the splits its launches and its merge use: those, or the tiled kernel's
+// fewer ones for the shapes only it and the general kernel take
+SplitPlan launch_splits(const kvssd_decode_desc& d, int units);
 
 // ---- general kernel: any head_dim <= 256, group size, GQA ratio, block size
 int launch_general(const DecodeArgs& a, const SplitPlan& plan, SplitPartials parts);
+
+// ---- tiled matrix-core kernel: the general kernel's fp32-grade arithmetic for head_dim 64 / 96 (INT4) / 128 / 256
+bool tile_supported(const kvssd_decode_desc& d);
+bool tile_aligned(const DecodeArgs& a);
+SplitPlan tile_splits(const kvssd_decode_desc& d, int units, const SplitPlan& most);
+int launch_tile(const DecodeArgs& a, const SplitPlan& plan, SplitPartials parts);
 
 // ---- matrix-core kernel: head_dim 128, group_size 32, bits 2/4
 bool mfma_supported(const kvssd_decode_desc& d, std::string* why);

@@ -1,6 +1,9 @@
 // General fused decode kernel: every shape the reference accepts
 // (head_dim <= 256, any group size with head_dim % group_size == 0, INT2/INT4,
-// any GQA ratio, any block_tokens), fp32 arithmetic on the VALU.
+// any GQA ratio, any block_tokens), fp32 arithmetic on the VALU.  It runs where
+// the tiled matrix-core kernel (decode_tile.hip, the same precision and 10-20
+// times its speed) does not apply: other head dims, more than 16 groups per
+// head, blocks that are no multiple of 16 tokens, unaligned arrays.
 //
 // Semantics: ReferenceAttentionBackend.run (src/kvssd/backends/reference.py:22-50)
 // and csrc/fused_decode.cu:12-90 (element addressing :50-56, GQA map :34).
@@ -197,8 +200,14 @@ SplitPlan plan_splits(const kvssd_decode_desc& d, int units) {
   return plan;
 }
 
+SplitPlan launch_splits(const kvssd_decode_desc& d, int units) {
+  const SplitPlan most = plan_splits(d, units);
+  return tile_supported(d) && !mfma_supported(d, nullptr) ? tile_splits(d, units, most) : most;
+}
+
 int launch_general(const DecodeArgs& a, const SplitPlan& plan, SplitPartials parts) {
   const kvssd_decode_desc& d = a.desc;
+  if (tile_supported(d) && tile_aligned(a)) return launch_tile(a, plan, parts);
   const int gq = d.query_heads / d.kv_heads;
   const int heads_per_chunk = gq < kMaxHeads ? gq : kMaxHeads;
   const int head_chunks = (gq + heads_per_chunk - 1) / heads_per_chunk;
