@@ -57,6 +57,15 @@ struct GatherParams {
   int32_t* status;
 };
 
+__device__ __forceinline__ int header_status(const uint32_t* hdr, const Layout& lay) {
+  if (hdr[0] != kMagic0 || hdr[1] != kMagic1 || hdr[2] != 1u) return 1;
+  if (hdr[6] != static_cast<uint32_t>(lay.bits) || hdr[7] != static_cast<uint32_t>(lay.block_tokens) ||
+      hdr[8] != static_cast<uint32_t>(lay.kv_heads) || hdr[9] != static_cast<uint32_t>(lay.head_dim) ||
+      hdr[10] != static_cast<uint32_t>(lay.group_size))
+    return 2;
+  return 0;
+}
+
 // one workgroup per record; status: 0 ok, 1 invalid header (magic / version),
 // 2 layout differs from the expected one, 3 payload length or CRC mismatch
 __global__ __launch_bounds__(kCrcThreads) void gather_records_kernel(GatherParams p) {
@@ -68,14 +77,7 @@ __global__ __launch_bounds__(kCrcThreads) void gather_records_kernel(GatherParam
   fill_crc_tables(tab);
   if (threadIdx.x < kHeaderBytes / 4) hdr[threadIdx.x] = reinterpret_cast<const uint32_t*>(rec)[threadIdx.x];
   __syncthreads();
-  int status = 0;
-  if (hdr[0] != kMagic0 || hdr[1] != kMagic1 || hdr[2] != 1u) {
-    status = 1;
-  } else if (hdr[6] != static_cast<uint32_t>(p.lay.bits) || hdr[7] != static_cast<uint32_t>(p.lay.block_tokens) ||
-             hdr[8] != static_cast<uint32_t>(p.lay.kv_heads) || hdr[9] != static_cast<uint32_t>(p.lay.head_dim) ||
-             hdr[10] != static_cast<uint32_t>(p.lay.group_size)) {
-    status = 2;
-  }
+  int status = header_status(hdr, p.lay);
   const int64_t s = p.lay.scale_bytes(), pb = p.lay.packed_bytes();
   const uint8_t* pay = rec + kHeaderBytes;
   copy_region(pay, p.sk + r * s, s);
@@ -98,29 +100,33 @@ __global__ __launch_bounds__(kCrcThreads) void gather_records_kernel(GatherParam
 }
 
 // chunked form of gather_records_kernel (same statuses), for layouts whose
-// four arrays are 16-byte multiples and 16-byte aligned destinations
-__global__ __launch_bounds__(kCrcThreads) void gather_chunked_kernel(GatherParams p, ChunkPlan c) {
+// four arrays are 16-byte multiples and 16-byte aligned destinations.  Each
+// thread takes its chunks four rows at a time, from memory to the arrays and
+// through the CRC, in at most 64 registers: two workgroups share a CU, and the
+// loads of some waves cover the matrix work of the others.
+__global__ __launch_bounds__(kCrcThreads, 8) void gather_chunked_kernel(GatherParams p, ChunkPlan c) {
   __shared__ ChunkLds lds;
   __shared__ uint32_t hdr[kHeaderBytes / 4];
   const int r = blockIdx.x;
   const uint8_t* rec = p.records + static_cast<int64_t>(r) * p.stride;
   const uint8_t* pay = rec + kHeaderBytes;
-  u32x4 v[kMaxRows];
-#pragma unroll
-  for (int j = 0; j < kMaxRows; ++j) {
-    v[j] = u32x4{0u, 0u, 0u, 0u};
-    if (j < c.rows) {
-      const int64_t o = chunk_offset(c, j);
-      if (o >= 0) v[j] = load16(pay + o);
-    }
-  }
   if (threadIdx.x < kHeaderBytes / 4) hdr[threadIdx.x] = reinterpret_cast<const uint32_t*>(rec)[threadIdx.x];
   if (p.verify) load_chunk_tables(lds);
+  __syncthreads();
   const int64_t sb = p.lay.scale_bytes(), pb = p.lay.packed_bytes();
+  uint32_t h = 0;
+  const int lead = (kGroupRows - c.rows % kGroupRows) % kGroupRows;  // zero rows of the first group
+  for (int j0 = -lead; j0 < c.rows; j0 += kGroupRows) {
+    u32x4 v[kGroupRows];
 #pragma unroll
-  for (int j = 0; j < kMaxRows; ++j) {
-    if (j < c.rows) {
-      const int64_t o = chunk_offset(c, j);
+    for (int j = 0; j < kGroupRows; ++j) {
+      v[j] = u32x4{0u, 0u, 0u, 0u};
+      const int64_t o = chunk_offset(c, j0 + j);
+      if (o >= 0) v[j] = load16(pay + o);
+    }
+#pragma unroll
+    for (int j = 0; j < kGroupRows; ++j) {
+      const int64_t o = chunk_offset(c, j0 + j);
       if (o >= 0) {
         uint8_t* dst;
         if (o < sb) dst = p.sk + r * sb + o;
@@ -130,28 +136,13 @@ __global__ __launch_bounds__(kCrcThreads) void gather_chunked_kernel(GatherParam
         *reinterpret_cast<u32x4*>(dst) = v[j];
       }
     }
+    if (p.verify) h = crc_group(lds, h, v, j0 < 0 ? -j0 : 0);
   }
-  __syncthreads();
-  int status = 0;
-  if (hdr[0] != kMagic0 || hdr[1] != kMagic1 || hdr[2] != 1u) {
-    status = 1;
-  } else if (hdr[6] != static_cast<uint32_t>(p.lay.bits) || hdr[7] != static_cast<uint32_t>(p.lay.block_tokens) ||
-             hdr[8] != static_cast<uint32_t>(p.lay.kv_heads) || hdr[9] != static_cast<uint32_t>(p.lay.head_dim) ||
-             hdr[10] != static_cast<uint32_t>(p.lay.group_size)) {
-    status = 2;
-  }
+  int status = header_status(hdr, p.lay);
   // status, p.verify and the header are the same in every thread, so the
   // fold's barriers are reached by the whole workgroup or by none of it
   if (p.verify && status == 0) {
-    if (hdr[11] != p.plan.len) {
-      status = 3;
-    } else {
-      uint32_t h = 0;
-#pragma unroll
-      for (int j = 0; j < kMaxRows; ++j)
-        if (j < c.rows) h = mul_stride(lds, h) ^ crc16_raw(lds, v[j]);
-      if (fold_chunks(lds, c, h) != hdr[12]) status = 3;
-    }
+    if (hdr[11] != p.plan.len || fold_chunks(lds, c, h) != hdr[12]) status = 3;
   }
   if (threadIdx.x == 0) {
     p.status[r] = status;
@@ -298,37 +289,45 @@ __global__ __launch_bounds__(256) void encode_payload_kernel(EncodeParams p) {
 }
 
 // phase 2: one workgroup per record -- CRC of the payload, header, padding.
-// CHUNKED: the payload is a 16-byte multiple of at most kMaxRows rows.
+// CHUNKED: the payload is a 16-byte multiple.
+struct WalkLds {
+  uint32_t tab[4][256];
+  uint32_t seg[kCrcThreads];
+};
+
 template <bool CHUNKED>
 __global__ __launch_bounds__(kCrcThreads) void encode_header_kernel(EncodeParams p, ChunkPlan c) {
-  __shared__ ChunkLds lds;
+  __shared__ union {
+    ChunkLds lds;
+    WalkLds walk;
+  } shared;
+  ChunkLds& lds = shared.lds;
+  WalkLds& walk = shared.walk;
   const Layout& L = p.lay;
   const int r = blockIdx.x;
   uint8_t* rec = p.records + static_cast<int64_t>(r) * L.record_bytes();
   uint32_t crc;
   if constexpr (CHUNKED) {
     const uint8_t* pay = rec + kHeaderBytes;
-    u32x4 v[kMaxRows];
-#pragma unroll
-    for (int j = 0; j < kMaxRows; ++j) {
-      v[j] = u32x4{0u, 0u, 0u, 0u};
-      if (j < c.rows) {
-        const int64_t o = chunk_offset(c, j);
-        if (o >= 0) v[j] = load16(pay + o);
-      }
-    }
     load_chunk_tables(lds);
     __syncthreads();
     uint32_t h = 0;
+    const int lead = (kGroupRows - c.rows % kGroupRows) % kGroupRows;
+    for (int j0 = -lead; j0 < c.rows; j0 += kGroupRows) {
+      u32x4 v[kGroupRows];
 #pragma unroll
-    for (int j = 0; j < kMaxRows; ++j)
-      if (j < c.rows) h = mul_stride(lds, h) ^ crc16_raw(lds, v[j]);
+      for (int j = 0; j < kGroupRows; ++j) {
+        v[j] = u32x4{0u, 0u, 0u, 0u};
+        const int64_t o = chunk_offset(c, j0 + j);
+        if (o >= 0) v[j] = load16(pay + o);
+      }
+      h = crc_group(lds, h, v, j0 < 0 ? -j0 : 0);
+    }
     crc = fold_chunks(lds, c, h);
   } else {
-    uint32_t(*tab)[256] = lds.slice;  // the first four slicing tables
-    fill_crc_tables(tab);
+    fill_crc_tables(walk.tab);
     __syncthreads();
-    crc = block_crc32(rec + kHeaderBytes, p.plan, tab, lds.seg);
+    crc = block_crc32(rec + kHeaderBytes, p.plan, walk.tab, walk.seg);
   }
   const int64_t start = static_cast<int64_t>(r) * L.block_tokens;
   const int64_t valid = p.tokens - start < L.block_tokens ? p.tokens - start : L.block_tokens;
@@ -367,10 +366,10 @@ __global__ __launch_bounds__(kCrcThreads) void encode_header_kernel(EncodeParams
 // the payload is never read back; the header and padding follow.
 struct FusedPlan {
   int rows_s, rows_c;  // rows of scale / code chunks
+  uint32_t x_codes;    // x^(8 * code bytes) mod P
 };
 
-constexpr int kMaxScaleRows = 4;  // scale region <= 64 KiB of LDS
-constexpr int kMaxCodeRows = 8;   // code chunks kept in registers for the CRC
+constexpr int kMaxScaleRows = kGroupRows;  // scale region <= 64 KiB of LDS, one group of rows
 
 template <typename T, int BITS>
 __global__ __launch_bounds__(kCrcThreads) void encode_fused_kernel(EncodeParams p, ChunkPlan c, FusedPlan f) {
@@ -386,12 +385,16 @@ __global__ __launch_bounds__(kCrcThreads) void encode_fused_kernel(EncodeParams 
   uint8_t* pay = rec + kHeaderBytes;
   const int64_t code0 = 2 * L.scale_bytes();
   load_chunk_tables(lds);
-  u32x4 code[kMaxCodeRows];
+  __syncthreads();  // the CRC matrices are in LDS
+  uint32_t h = 0;
+  const int lead = (kGroupRows - f.rows_c % kGroupRows) % kGroupRows;  // zero rows of the first group
+  for (int k0 = -lead; k0 < f.rows_c; k0 += kGroupRows) {
+    u32x4 code[kGroupRows];
 #pragma unroll
-  for (int k = 0; k < kMaxCodeRows; ++k) {
-    code[k] = u32x4{0u, 0u, 0u, 0u};
-    if (k < f.rows_c) {
-      const int64_t chunk = static_cast<int64_t>(k) * kCrcThreads + tid;  // within the code region
+    for (int k = 0; k < kGroupRows; ++k) {
+      code[k] = u32x4{0u, 0u, 0u, 0u};
+      if (k0 + k < 0) continue;
+      const int64_t chunk = static_cast<int64_t>(k0 + k) * kCrcThreads + tid;  // within the code region
       uint32_t w[4];
 #pragma unroll
       for (int i = 0; i < kGroupsPerChunk; ++i) {
@@ -413,22 +416,25 @@ __global__ __launch_bounds__(kCrcThreads) void encode_fused_kernel(EncodeParams 
       code[k] = u32x4{w[0], w[1], w[2], w[3]};
       __builtin_memcpy(__builtin_assume_aligned(pay + code0 + chunk * kChunkBytes, 4), &code[k], kChunkBytes);
     }
+    h = crc_group(lds, h, code, k0 < 0 ? -k0 : 0);
   }
-  __syncthreads();  // every scale is in LDS (and the CRC tables)
-  uint32_t h = 0;
+  __syncthreads();  // every scale is in LDS
+  u32x4 v[kGroupRows];
 #pragma unroll
-  for (int j = 0; j < kMaxScaleRows; ++j) {
-    if (j < f.rows_s) {
-      const int64_t chunk = static_cast<int64_t>(j) * kCrcThreads + tid;
-      const u32x4 v = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint8_t*>(scales) + chunk * kChunkBytes);
-      __builtin_memcpy(__builtin_assume_aligned(pay + chunk * kChunkBytes, 4), &v, kChunkBytes);
-      h = mul_stride(lds, h) ^ crc16_raw(lds, v);
+  for (int j = 0; j < kGroupRows; ++j) {
+    v[j] = u32x4{0u, 0u, 0u, 0u};
+    const int row = j + f.rows_s - kGroupRows;
+    if (row >= 0) {
+      const int64_t chunk = static_cast<int64_t>(row) * kCrcThreads + tid;
+      v[j] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint8_t*>(scales) + chunk * kChunkBytes);
+      __builtin_memcpy(__builtin_assume_aligned(pay + chunk * kChunkBytes, 4), &v[j], kChunkBytes);
     }
   }
-#pragma unroll
-  for (int k = 0; k < kMaxCodeRows; ++k)
-    if (k < f.rows_c) h = mul_stride(lds, h) ^ crc16_raw(lds, code[k]);
-  const uint32_t crc = fold_chunks(lds, c, h);
+  const uint32_t hs = crc_group(lds, 0u, v, kGroupRows - f.rows_s);
+  // the scales come before the codes in the message
+  const uint32_t raw_s = fold_columns(lds, kPosTables.chunk, hs);
+  const uint32_t raw_c = fold_columns(lds, kPosTables.chunk, h);
+  const uint32_t crc = crc_from_raw(c.x_len, gf_mul_dev(f.x_codes, raw_s) ^ raw_c);
   const int64_t start = static_cast<int64_t>(r) * L.block_tokens;
   const int64_t valid = p.tokens - start < L.block_tokens ? p.tokens - start : L.block_tokens;
   if (tid < kHeaderBytes / 4) {
@@ -461,15 +467,13 @@ bool fused_layout(const Layout& L, FusedPlan* f) {
   if (L.group_size != kRegGroup || sr % kStrideBytes || cr % kStrideBytes) return false;
   f->rows_s = static_cast<int>(sr / kStrideBytes);
   f->rows_c = static_cast<int>(cr / kStrideBytes);
-  return f->rows_s >= 1 && f->rows_s <= kMaxScaleRows && f->rows_c >= 1 && f->rows_c <= kMaxCodeRows &&
-         f->rows_s + f->rows_c <= kMaxRows;
+  f->x_codes = x_pow_bytes(static_cast<uint64_t>(cr));
+  return f->rows_s >= 1 && f->rows_s <= kMaxScaleRows && f->rows_c >= 1;
 }
 
-// the chunked CRC / gather form applies: all four arrays 16-byte multiples and
-// the payload at most kMaxRows rows of chunks
+// the chunked CRC / gather form applies: all four arrays 16-byte multiples
 bool chunked_layout(const Layout& L) {
-  return L.scale_bytes() % kChunkBytes == 0 && L.packed_bytes() % kChunkBytes == 0 &&
-         L.payload_bytes() <= static_cast<int64_t>(kMaxRows) * kStrideBytes;
+  return L.scale_bytes() % kChunkBytes == 0 && L.packed_bytes() % kChunkBytes == 0;
 }
 
 int check_layout(const kvssd_record_layout* l, Layout* out) {
@@ -652,7 +656,7 @@ int launch_encode_records(const kvssd_record_layout* layout, int dtype, const vo
       return arg_error("quantization input must be floating point");
   }
   if (int rc = hip_status(hipGetLastError(), "encode_records launch")) return rc;
-  if (len % kChunkBytes == 0 && c.rows <= kMaxRows) {
+  if (len % kChunkBytes == 0) {
     hipLaunchKernelGGL(encode_header_kernel<true>, dim3(static_cast<unsigned>(p.n)), dim3(kCrcThreads), 0, stream, p, c);
   } else {
     hipLaunchKernelGGL(encode_header_kernel<false>, dim3(static_cast<unsigned>(p.n)), dim3(kCrcThreads), 0, stream, p, c);

@@ -114,7 +114,8 @@ __global__ __launch_bounds__(kCrcThreads) void vllm_rows_kernel(const uint8_t* _
     }
   }
   __syncthreads();  // tables in LDS
-  const uint32_t h = crc16_raw(lds, v);
+  const u32x4 rows[kGroupRows] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}, v};
+  const uint32_t h = crc_group(lds, 0u, rows, kGroupRows - 1);
   if constexpr (BITS != 0) {
     const int64_t q0 = o - sh.scale_bytes;  // first byte of the chunk in the packed region
     if (q0 >= 0) {
@@ -133,7 +134,7 @@ __global__ __launch_bounds__(kCrcThreads) void vllm_rows_kernel(const uint8_t* _
       }
     }
   }
-  const uint32_t raw = fold_pos(lds, kPosTables.chunk, h);
+  const uint32_t raw = fold_columns(lds, kPosTables.chunk, h);
   if (threadIdx.x == 0) parts[blockIdx.x] = raw;
 }
 
@@ -147,11 +148,11 @@ __global__ __launch_bounds__(kCrcThreads) void vllm_combine_kernel(const uint32_
                                                                    uint32_t hdr3, uint32_t hdr4, int64_t record_bytes,
                                                                    uint32_t expected, int32_t* __restrict__ status,
                                                                    uint32_t* __restrict__ crc_out) {
-  __shared__ ChunkLds lds;
+  __shared__ uint32_t seg[kCrcThreads / 64];
   const int t = threadIdx.x;
   const int lead = kCrcThreads - pl.rows;  // leading zero rows leave the raw register unchanged
   const uint32_t h = t >= lead ? parts[t - lead] : 0u;
-  const uint32_t crc = crc_from_raw(pl.x_len, fold_pos(lds, kPosTables.row, h));
+  const uint32_t crc = crc_from_raw(pl.x_len, fold_pos(seg, kPosTables.row, h));
   if constexpr (ENCODE) {
     if (t < kVHeader / 4) {
       uint32_t w = 0;

@@ -226,3 +226,21 @@ def test_quantize_unaligned_source_matches(cuda_device, bits):
     packed, scales = oracle_quantize(x, bits, 32)
     assert torch.equal(a.packed, b.packed) and np.array_equal(a.packed.cpu().numpy(), packed)
     assert np.array_equal(a.scales.cpu().numpy().view(np.uint16), scales.view(np.uint16))
+
+
+@pytest.mark.parametrize("block_tokens", [1, 127, 128, 129, 512, 513, 1300, 2433])
+def test_chunked_crc_row_edges(cuda_device, block_tokens):
+    # 128 payload bytes a token: part of a row of 1024 16-byte chunks, one row, four (a whole
+    # group of rows), one chunk more, and more than 16 rows; CRC values are zlib's, and one
+    # flipped bit at either end or in the middle of the payload is seen
+    spec = CacheSpec(1, 1, 96, block_tokens, 4, 12)
+    gen = torch.Generator().manual_seed(block_tokens)
+    k = torch.randn(5 * block_tokens, 1, 96, generator=gen).half().to(cuda_device)
+    recs, crcs = R.encode_records(k, k.flip(0), spec, 0)
+    n = 128 * block_tokens
+    host = recs.cpu().numpy()
+    assert crcs.tolist() == [zlib.crc32(r[52 : 52 + n].tobytes()) for r in host]
+    for i, (byte, bit) in enumerate([(0, 0), (n // 2, 3), (n - 1, 7), (n // 3, 5)]):
+        recs[i, 52 + byte] ^= 1 << bit
+    *_, status = R.gather_records(recs.view(-1), spec, 5)
+    assert status.tolist() == [R.BAD_CRC] * 4 + [R.OK]
