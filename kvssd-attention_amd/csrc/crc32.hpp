@@ -91,9 +91,11 @@ __device__ const CrcTables kCrcTables = make_crc_tables();
 // Position multipliers of the chunked form: chunk[t] = x^(8 * 16 * (1023 - t)),
 // row[t] = x^(8 * 16384 * (1023 - t)) -- the shift of piece t of 1024 equal
 // pieces to the end of the message they form.
+// word[t] = that of the last dword of thread t's column in the dword layout (below).
 struct PosTables {
   uint32_t chunk[kCrcThreads];
   uint32_t row[kCrcThreads];
+  uint32_t word[kCrcThreads];
 };
 
 constexpr PosTables make_pos_tables() {
@@ -105,6 +107,9 @@ constexpr PosTables make_pos_tables() {
     p.chunk[t - 1] = gf_mul(p.chunk[t], sc);
     p.row[t - 1] = gf_mul(p.row[t], sr);
   }
+  const uint32_t sw = x_pow_bytes(4);
+  for (int t = kCrcThreads - 1; t >= 0; --t)
+    p.word[t] = (t & 31) == 31 ? p.chunk[t | 63] : gf_mul(p.word[t + 1], sw);
   return p;
 }
 
@@ -189,8 +194,11 @@ constexpr int kGroupRows = 4;  // rows of chunks between two parity steps
 // Matrices of the chunked form as A operands, one u32x4 per lane: lane (r, half)
 // holds bit r of the CRC contributions of 32 message bits, nibble i of dword p
 // that of bit 4 i + p.  data[j][w]: dword w of a chunk in row j of a group, in
-// lane half 0 (32 chunks before half 1's).  carry: the column's raw CRC before
-// the group, bits split over the halves as the parities are.
+// lane half 0 (32 chunks before half 1's).  In the dword layout a wave's 1 KiB
+// of a row is four runs of 64 dwords instead, lane l holding dword l of each:
+// data[j][w] is run w, and half 0's dword lies 32 dwords before half 1's.
+// carry: the column's raw CRC before the group, bits split over the halves as
+// the parities are.
 struct BitMatrices {
   uint32_t data[kGroupRows][4][64][4];
   uint32_t carry[64][4];
@@ -201,17 +209,20 @@ constexpr uint32_t kHalfBits = 0x0F0F0F0Fu;
 
 constexpr uint32_t fp4_factor(int plane) { return plane == 0 ? 4u : plane == 1 ? 2u : 1u; }  // 2, 1, 0.5
 
-constexpr BitMatrices make_bit_matrices() {
+constexpr BitMatrices make_bit_matrices(bool words) {
   BitMatrices m{};
   uint32_t row_pow[kGroupRows] = {};
   row_pow[kGroupRows - 1] = 0x80000000u;  // x^0
   const uint32_t stride = x_pow_bytes(kStrideBytes);
   for (int j = kGroupRows - 1; j > 0; --j) row_pow[j - 1] = gf_mul(row_pow[j], stride);
   const uint32_t over = gf_mul(row_pow[0], stride);  // a whole group of rows
-  const uint32_t half_pow = x_pow_bytes(32 * kChunkBytes);
-  uint32_t byte_pow[kChunkBytes] = {};  // byte b of a chunk, to the chunk's end (its own 8 shifts with it)
+  const uint32_t half_pow = x_pow_bytes(32 * (words ? 4 : kChunkBytes));
+  // byte b of dword w, to the end of the chunk (the last run): its own 8 shifts and the bytes after it
+  uint32_t byte_pow[kChunkBytes] = {};
   byte_pow[kChunkBytes - 1] = 0x00800000u;
-  for (int b = kChunkBytes - 1; b > 0; --b) byte_pow[b - 1] = gf_mul(byte_pow[b], 0x00800000u);
+  const uint32_t run = words ? x_pow_bytes(4 * 64) : x_pow_bytes(4);
+  for (int b = kChunkBytes - 1; b > 0; --b)
+    byte_pow[b - 1] = (b & 3) != 0 ? gf_mul(byte_pow[b], 0x00800000u) : gf_mul(byte_pow[b + 3], run);
   for (int bit = 0; bit < 32; ++bit) {
     const int plane = bit & 3;
     const uint32_t value = fp4_factor(plane) << (4 * (bit >> 2));
@@ -234,7 +245,8 @@ constexpr BitMatrices make_bit_matrices() {
   return m;
 }
 
-__device__ const BitMatrices kBitMatrices = make_bit_matrices();
+__device__ const BitMatrices kBitMatrices = make_bit_matrices(false);
+__device__ const BitMatrices kWordMatrices = make_bit_matrices(true);
 
 struct ChunkLds {
   u32x4 data[kGroupRows][4][64];
@@ -242,8 +254,8 @@ struct ChunkLds {
   uint32_t seg[kCrcThreads / 64];
 };
 
-__device__ __forceinline__ void load_chunk_tables(ChunkLds& l) {
-  const u32x4* src = reinterpret_cast<const u32x4*>(&kBitMatrices);
+__device__ __forceinline__ void load_chunk_tables(ChunkLds& l, const BitMatrices& m = kBitMatrices) {
+  const u32x4* src = reinterpret_cast<const u32x4*>(&m);
   u32x4* dst = &l.data[0][0][0];  // data then carry: 1024 + 64 entries
   const u32x4 v = src[threadIdx.x];
   if (threadIdx.x < 64) dst[kCrcThreads + threadIdx.x] = src[kCrcThreads + threadIdx.x];
@@ -268,22 +280,24 @@ __device__ __forceinline__ f32x16 count_bits(u32x4 a, uint32_t x, f32x16 acc) {
   return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(A, B, acc, 4, 4, 0, 127, 0, 127);  // fp4, block scales 2^0
 }
 
-// Column state h (this lane half's bits of the column's raw CRC) carried over a
-// group of rows; row j of the group is v[j], rows before `first` are zeros.
-// Every lane of the wave takes part.
-__device__ __forceinline__ uint32_t crc_group(const ChunkLds& l, uint32_t h, const u32x4 (&v)[kGroupRows], int first) {
-  const int lane = threadIdx.x & 63;
+// Counts of a group of rows, from the column state h (this lane half's bits of
+// the column's raw CRC) carried over it.  Every lane of the wave takes part.
+__device__ __forceinline__ f32x16 crc_begin(const ChunkLds& l, uint32_t h) {
   f32x16 acc;
 #pragma unroll
   for (int i = 0; i < 16; ++i) acc[i] = 8388608.0f;  // 2^23: a count's parity is the lowest bit
-  acc = count_bits(l.carry[lane], h, acc);
+  return count_bits(l.carry[threadIdx.x & 63], h, acc);
+}
+
+// ... with row j of the group
+__device__ __forceinline__ f32x16 crc_row(const ChunkLds& l, f32x16 acc, int j, u32x4 v) {
 #pragma unroll
-  for (int j = 0; j < kGroupRows; ++j) {
-    if (j >= first) {
-#pragma unroll
-      for (int w = 0; w < 4; ++w) acc = count_bits(l.data[j][w][lane], v[j][w], acc);
-    }
-  }
+  for (int w = 0; w < 4; ++w) acc = count_bits(l.data[j][w][threadIdx.x & 63], v[w], acc);
+  return acc;
+}
+
+// ... and the column state after it
+__device__ __forceinline__ uint32_t crc_end(f32x16 acc) {
   // register i holds CRC bit 8 (i / 4) + i % 4, + 4 in lane half 1
   uint32_t p = 0;
 #pragma unroll
@@ -291,7 +305,16 @@ __device__ __forceinline__ uint32_t crc_group(const ChunkLds& l, uint32_t h, con
     const float count = acc[i];  // (a bit cast of acc[i] itself reads acc[0])
     p |= (__builtin_bit_cast(uint32_t, count) & 1u) << (8 * (i >> 2) + (i & 3));
   }
-  return p << ((lane >> 5) * 4);
+  return p << (((threadIdx.x & 63) >> 5) * 4);
+}
+
+// A group of rows v, the first `first` of them zeros.
+__device__ __forceinline__ uint32_t crc_group(const ChunkLds& l, uint32_t h, const u32x4 (&v)[kGroupRows], int first) {
+  f32x16 acc = crc_begin(l, h);
+#pragma unroll
+  for (int j = 0; j < kGroupRows; ++j)
+    if (j >= first) acc = crc_row(l, acc, j, v[j]);
+  return crc_end(acc);
 }
 
 // Chunk geometry of a payload of `len` bytes (a multiple of 16): `rows` rows of

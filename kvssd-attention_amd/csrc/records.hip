@@ -195,6 +195,61 @@ struct GroupWords {
   uint16_t scale;                     // fp16 bits
 };
 
+// A word of codes, low bits first: clamp(rint(x / s32), -mid, mid - 1) + mid
+// with x / s32 rounded as IEEE division does, |x| <= (mid - 1) s32 (1 + 2^-23) or
+// x NaN (code 0).  Two roundings around a reciprocal stand in for the division
+// (~12 instructions a value):
+// * 16-bit values: q = x r, then q + (x - q s32) r, off x / s32 by at most
+//   2^-46 relative before its own rounding.  The codes could then differ only
+//   where x / s32 lies that close to half an ulp off some k + 0.5; with x and
+//   the group's largest value in 16 bits, both quotients in question are at
+//   least 2^-38 apart (checked over every such pair in float16 and bfloat16);
+// * 32-bit values: q = x r is off by less than 2^-19, so that its nearest
+//   integer is right unless q lies within 2^-18 of some k + 0.5; then, and for
+//   scales whose reciprocal is subnormal or zero, the division itself.
+template <typename T, int BITS>
+__device__ __forceinline__ uint32_t code_word(const float (&x)[32 / BITS], float s32) {
+  constexpr int kCodes = 32 / BITS;
+  constexpr float mid = static_cast<float>(1 << (BITS - 1));
+  float c[kCodes];
+  bool done = false;
+  if (s32 < 0x1p120f) {
+    const float r0 = __builtin_amdgcn_rcpf(s32);
+    const float r = __builtin_fmaf(__builtin_fmaf(-s32, r0, 1.0f), r0, r0);
+    float off = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kCodes; ++i) {
+      float q = x[i] * r;
+      if constexpr (sizeof(T) == 2) q = __builtin_fmaf(__builtin_fmaf(-q, s32, x[i]), r, q);
+      const float n = rintf(q);
+      if constexpr (sizeof(T) != 2) off = fmaxf(off, fabsf(q - n));
+      c[i] = fminf(fmaxf(n, -mid), mid - 1.0f);
+    }
+    done = sizeof(T) == 2 || off < 0.5f - 0x1p-18f;
+  }
+  if (!done) {
+#pragma unroll
+    for (int i = 0; i < kCodes; ++i) c[i] = fminf(fmaxf(rintf(x[i] / s32), -mid), mid - 1.0f);
+  }
+  // 16 bits at a time as an exact float sum
+  uint32_t half[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    constexpr int n = kCodes / 2;
+    float t = c[k * n + n - 1] + mid;
+#pragma unroll
+    for (int i = n - 2; i >= 0; --i) t = __builtin_fmaf(t, static_cast<float>(1 << BITS), c[k * n + i] + mid);
+    half[k] = static_cast<uint32_t>(t);
+  }
+  return half[0] | (half[1] << 16);
+}
+
+// max(amax, 1e-8) / (mid - 1), IEEE
+template <int BITS>
+__device__ __forceinline__ float group_scale(float amax) {
+  return fmaxf(amax, 1e-8f) / static_cast<float>((1 << (BITS - 1)) - 1);
+}
+
 template <typename T, int BITS>
 __device__ __forceinline__ GroupWords<BITS> quantize_group_words(const T* src) {
   float x[kRegGroup];
@@ -210,15 +265,14 @@ __device__ __forceinline__ GroupWords<BITS> quantize_group_words(const T* src) {
   float amax = 0.0f;
 #pragma unroll
   for (int i = 0; i < kRegGroup; ++i) amax = fmaxf(amax, fabsf(x[i]));
-  constexpr int mid = 1 << (BITS - 1);
-  const float s32 = fmaxf(amax, 1e-8f) / static_cast<float>(mid - 1);
+  const float s32 = group_scale<BITS>(amax);
   GroupWords<BITS> g;
 #pragma unroll
-  for (int k = 0; k < kRegGroup * BITS / 32; ++k) g.w[k] = 0;
+  for (int k = 0; k < BITS; ++k) {
+    float part[32 / BITS];
 #pragma unroll
-  for (int i = 0; i < kRegGroup; ++i) {
-    const float c = fminf(fmaxf(rintf(x[i] / s32), static_cast<float>(-mid)), static_cast<float>(mid - 1));
-    g.w[(i * BITS) >> 5] |= static_cast<uint32_t>(static_cast<int>(c) + mid) << ((i * BITS) & 31);
+    for (int i = 0; i < 32 / BITS; ++i) part[i] = x[k * (32 / BITS) + i];
+    g.w[k] = code_word<T, BITS>(part, s32);
   }
   g.scale = __builtin_bit_cast(uint16_t, static_cast<_Float16>(s32));
   return g;
@@ -354,16 +408,19 @@ __global__ __launch_bounds__(kCrcThreads) void encode_header_kernel(EncodeParams
   if (threadIdx.x == 0) p.crcs[r] = crc;
 }
 
-// One kernel for the common layout (group size 32 in registers, the scale
-// region [Ks | Vs] and the code region [Kc | Vc] each a whole number of
-// 16 KiB rows of the chunked CRC form, so no virtual zeros): one workgroup of
-// 1024 threads per record.  Thread t owns code chunks t, t + 1024, ... (rows
-// rs .. rows - 1 of the chunked form): it quantises their groups (one INT4
-// group or two INT2 groups per 16-byte chunk), stores each chunk, keeps it
-// in registers and puts the scales into an LDS copy of the scale region.
-// After a barrier it stores and reads back its scale chunks (rows 0 .. rs - 1)
-// from LDS and folds the record's CRC-32 from registers as the gather does, so
-// the payload is never read back; the header and padding follow.
+// One kernel for the common layout (group size 32, the scale region [Ks | Vs]
+// and the code region [Kc | Vc] each a whole number of 16 KiB rows of the
+// chunked CRC form, so no virtual zeros): one workgroup of 1024 threads per
+// record.  A record's codes are those of its keys, then its values, in memory
+// order, so wave w of code row k takes the 1 KiB piece 16 k + w as four runs of
+// 64 words: a lane reads the 8 (INT4) or 16 (INT2) values of its word, a group
+// is 4 or 2 lanes, loads and stores are contiguous over the wave, and the words
+// go through the CRC in its dword layout as they are made.  The scales collect
+// in LDS; after a barrier they are stored and take a CRC of their own, moved
+// before the codes' by one multiply, so the payload is never read back.
+// Measured (1,024 records of 8 kv heads, head_dim 128, bfloat16, 688 MB moved):
+// a lane a group, reading 64 bytes of its own, and IEEE divisions 222 us, 178
+// us in this form.
 struct FusedPlan {
   int rows_s, rows_c;  // rows of scale / code chunks
   uint32_t x_codes;    // x^(8 * code bytes) mod P
@@ -371,52 +428,95 @@ struct FusedPlan {
 
 constexpr int kMaxScaleRows = kGroupRows;  // scale region <= 64 KiB of LDS, one group of rows
 
+// largest of v over the BITS lanes (4 or 2) that share a group
+template <int BITS>
+__device__ __forceinline__ float group_max(float v) {
+  v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true)));
+  if constexpr (BITS == 4)
+    v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, true)));
+  return v;
+}
+
 template <typename T, int BITS>
 __global__ __launch_bounds__(kCrcThreads) void encode_fused_kernel(EncodeParams p, ChunkPlan c, FusedPlan f) {
   __shared__ ChunkLds lds;
-  __shared__ __attribute__((aligned(16))) uint16_t scales[kMaxScaleRows * kStrideBytes / 2];
-  constexpr int kGroupsPerChunk = 4 / BITS;  // 32-value groups in 16 bytes of codes
+  extern __shared__ __attribute__((aligned(16))) uint16_t scales[];  // the record's scale region
+  constexpr int kVals = 32 / BITS;                                   // values of a word of codes
+  constexpr int kRunBytes = 64 * 4;
+  constexpr int kRaw = kVals * static_cast<int>(sizeof(T)) / 4;      // dwords of those values
+  constexpr int kAhead = kRaw <= 4 ? 4 : kRaw <= 8 ? 2 : 1;          // runs loaded at a time
   const Layout& L = p.lay;
   const int r = blockIdx.x;
   const int tid = threadIdx.x;
-  const int G = L.head_dim / kRegGroup;
-  const int64_t per_array = static_cast<int64_t>(L.block_tokens) * L.kv_heads * G;  // groups per array
+  const int lane = tid & 63;
   uint8_t* rec = p.records + static_cast<int64_t>(r) * L.record_bytes();
   uint8_t* pay = rec + kHeaderBytes;
-  const int64_t code0 = 2 * L.scale_bytes();
-  load_chunk_tables(lds);
+  const int64_t code0 = 2 * L.scale_bytes(), array = L.packed_bytes();
+  // the record's first value of keys and of values, and how many follow before the last token's end
+  const int64_t block = static_cast<int64_t>(L.block_tokens) * L.kv_heads * L.head_dim;
+  const int64_t left = p.tokens * L.kv_heads * L.head_dim - r * block;
+  // the values of runs u0 .. u0 + kAhead - 1 of code row k's piece
+  auto piece_of = [&](int k) { return (static_cast<int64_t>(k) * kCrcThreads + (tid & ~63)) * kChunkBytes; };
+  auto load_runs = [&](int k, int u0, uint32_t (&raw)[kAhead][kRaw]) {
+    // codes of keys or of values (arrays are whole pieces)
+    const int64_t piece = piece_of(k);
+    const bool is_v = piece >= array;
+    const T* base = static_cast<const T*>(is_v ? p.values : p.keys) + r * block;
+    const int64_t at = (is_v ? piece - array : piece) * (8 / BITS) + lane * kVals;  // of the block's values
+#pragma unroll
+    for (int a = 0; a < kAhead; ++a) {
+      const int64_t e = at + (u0 + a) * 64 * kVals;
+      const bool in = e < left;
+      __builtin_memcpy(raw[a], __builtin_assume_aligned(base + (in ? e : 0), 16), sizeof(raw[a]));
+#pragma unroll
+      for (int i = 0; i < kRaw; ++i) raw[a][i] = in ? raw[a][i] : 0u;  // tokens past the end are zeros
+    }
+  };
+  uint32_t next[kAhead][kRaw];
+  load_runs(0, 0, next);
+  load_chunk_tables(lds, kWordMatrices);
   __syncthreads();  // the CRC matrices are in LDS
   uint32_t h = 0;
   const int lead = (kGroupRows - f.rows_c % kGroupRows) % kGroupRows;  // zero rows of the first group
   for (int k0 = -lead; k0 < f.rows_c; k0 += kGroupRows) {
-    u32x4 code[kGroupRows];
+    f32x16 acc = crc_begin(lds, h);
+#pragma unroll 1
+    for (int j = k0 < 0 ? -k0 : 0; j < kGroupRows; ++j) {
+      const int k = k0 + j;
+      const int64_t piece = piece_of(k);
+      u32x4 words;
 #pragma unroll
-    for (int k = 0; k < kGroupRows; ++k) {
-      code[k] = u32x4{0u, 0u, 0u, 0u};
-      if (k0 + k < 0) continue;
-      const int64_t chunk = static_cast<int64_t>(k0 + k) * kCrcThreads + tid;  // within the code region
-      uint32_t w[4];
+      for (int u0 = 0; u0 < 4; u0 += kAhead) {
+        uint32_t raw[kAhead][kRaw];
+        __builtin_memcpy(raw, next, sizeof(raw));
+        // the next runs' loads are in flight while these are quantised
+        if (u0 + kAhead < 4) load_runs(k, u0 + kAhead, next);
+        else if (k + 1 < f.rows_c) load_runs(k + 1, 0, next);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < kGroupsPerChunk; ++i) {
-        const int64_t q = chunk * kGroupsPerChunk + i;  // over [K groups | V groups]
-        const bool is_v = q >= per_array;
-        const int64_t qa = is_v ? q - per_array : q;
-        const int64_t row = qa / G;  // token * kv_heads + head within the block
-        const int gi = static_cast<int>(qa % G);
-        const int64_t token = static_cast<int64_t>(r) * L.block_tokens + row / L.kv_heads;
-        const T* base = static_cast<const T*>(is_v ? p.values : p.keys);
-        const T* src =
-            token < p.tokens ? base + (token * L.kv_heads + row % L.kv_heads) * L.head_dim + gi * kRegGroup : nullptr;
-        const GroupWords<BITS> g = quantize_group_words<T, BITS>(src);
-        constexpr int kWords = kRegGroup * BITS / 32;
+        for (int a = 0; a < kAhead; ++a) {
+          const int u = u0 + a;
+          T v[kVals];
+          __builtin_memcpy(v, raw[a], sizeof(v));
+          float x[kVals], amax = 0.0f;
 #pragma unroll
-        for (int k2 = 0; k2 < kWords; ++k2) w[i * kWords + k2] = g.w[k2];
-        scales[q] = g.scale;
+          for (int i = 0; i < kVals; ++i) {
+            x[i] = to_f32(v[i]);
+            amax = fmaxf(amax, fabsf(x[i]));
+          }
+          const float s32 = group_scale<BITS>(group_max<BITS>(amax));
+          const uint32_t word = code_word<T, BITS>(x, s32);
+          words[u] = word;
+          if ((lane & (BITS - 1)) == 0)
+            scales[piece / (4 * BITS) + u * (64 / BITS) + lane / BITS] =
+                __builtin_bit_cast(uint16_t, static_cast<_Float16>(s32));
+          __builtin_memcpy(__builtin_assume_aligned(pay + code0 + piece + u * kRunBytes + 4 * lane, 4), &word, 4);
+          __builtin_amdgcn_sched_barrier(0);  // (runs quantised side by side would not fit the registers)
+        }
       }
-      code[k] = u32x4{w[0], w[1], w[2], w[3]};
-      __builtin_memcpy(__builtin_assume_aligned(pay + code0 + chunk * kChunkBytes, 4), &code[k], kChunkBytes);
+      acc = crc_row(lds, acc, j, words);
     }
-    h = crc_group(lds, h, code, k0 < 0 ? -k0 : 0);
+    h = crc_end(acc);
   }
   __syncthreads();  // every scale is in LDS
   u32x4 v[kGroupRows];
@@ -425,15 +525,19 @@ __global__ __launch_bounds__(kCrcThreads) void encode_fused_kernel(EncodeParams 
     v[j] = u32x4{0u, 0u, 0u, 0u};
     const int row = j + f.rows_s - kGroupRows;
     if (row >= 0) {
-      const int64_t chunk = static_cast<int64_t>(row) * kCrcThreads + tid;
-      v[j] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint8_t*>(scales) + chunk * kChunkBytes);
-      __builtin_memcpy(__builtin_assume_aligned(pay + chunk * kChunkBytes, 4), &v[j], kChunkBytes);
+      const int64_t piece = (static_cast<int64_t>(row) * kCrcThreads + (tid & ~63)) * kChunkBytes;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t word = reinterpret_cast<const uint32_t*>(scales)[piece / 4 + u * 64 + lane];
+        __builtin_memcpy(__builtin_assume_aligned(pay + piece + u * kRunBytes + 4 * lane, 4), &word, 4);
+        v[j][u] = word;
+      }
     }
   }
   const uint32_t hs = crc_group(lds, 0u, v, kGroupRows - f.rows_s);
   // the scales come before the codes in the message
-  const uint32_t raw_s = fold_columns(lds, kPosTables.chunk, hs);
-  const uint32_t raw_c = fold_columns(lds, kPosTables.chunk, h);
+  const uint32_t raw_s = fold_columns(lds, kPosTables.word, hs);
+  const uint32_t raw_c = fold_columns(lds, kPosTables.word, h);
   const uint32_t crc = crc_from_raw(c.x_len, gf_mul_dev(f.x_codes, raw_s) ^ raw_c);
   const int64_t start = static_cast<int64_t>(r) * L.block_tokens;
   const int64_t valid = p.tokens - start < L.block_tokens ? p.tokens - start : L.block_tokens;
@@ -512,10 +616,11 @@ void launch_quantize_t(const void* x, int64_t groups, int group_size, int bits, 
 template <typename T>
 void launch_fused_t(const EncodeParams& p, const ChunkPlan& c, const FusedPlan& f, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(p.n));
+  const size_t scale_lds = static_cast<size_t>(2 * p.lay.scale_bytes());
   if (p.lay.bits == 4)
-    hipLaunchKernelGGL((encode_fused_kernel<T, 4>), grid, dim3(kCrcThreads), 0, s, p, c, f);
+    hipLaunchKernelGGL((encode_fused_kernel<T, 4>), grid, dim3(kCrcThreads), scale_lds, s, p, c, f);
   else
-    hipLaunchKernelGGL((encode_fused_kernel<T, 2>), grid, dim3(kCrcThreads), 0, s, p, c, f);
+    hipLaunchKernelGGL((encode_fused_kernel<T, 2>), grid, dim3(kCrcThreads), scale_lds, s, p, c, f);
 }
 
 template <typename T>

@@ -244,3 +244,37 @@ def test_chunked_crc_row_edges(cuda_device, block_tokens):
         recs[i, 52 + byte] ^= 1 << bit
     *_, status = R.gather_records(recs.view(-1), spec, 5)
     assert status.tolist() == [R.BAD_CRC] * 4 + [R.OK]
+
+
+@pytest.mark.parametrize("bits", [2, 4])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_quantize_around_ties(cuda_device, bits, dtype):
+    # values next to every k + 0.5 of groups with many different largest values, scales whose
+    # reciprocal is subnormal among them: where a reciprocal could stand in wrongly for the
+    # division; through the quantiser and through whole records, with the oracle's codes
+    rng = np.random.default_rng(bits)
+    top = (1 << (bits - 1)) - 1
+    amax = rng.uniform(1.0, 2.0, 2048) * 2.0 ** rng.integers(-12, 14, 2048)
+    if dtype != torch.float16:
+        amax[:64] = rng.uniform(1.0, 2.0, 64) * 1.5e38
+    amax = torch.from_numpy(amax).to(dtype)
+    s32 = amax.float() / top
+    ties = (torch.arange(32) % (2 * top) - top + 0.5) * s32[:, None]
+    step = torch.tensor([0.0, 1.0, -1.0, 2.0])[torch.arange(32) // 8]
+    x = (ties * (1 + step * torch.finfo(dtype).eps)).to(dtype)
+    x = torch.minimum(torch.maximum(x, -amax[:, None]), amax[:, None])
+    x[:, 31] = amax
+    x = x.reshape(-1, 128)  # 512 rows of four groups
+    packed, scales = oracle_quantize(x, bits, 32)
+    q = R.quantize(x.to(cuda_device), bits, 32)
+    assert np.array_equal(q.packed.cpu().numpy(), packed)
+    assert np.array_equal(q.scales.cpu().numpy().view(np.uint16), scales.view(np.uint16))
+    # one block of 128 tokens x 8 heads: the one-kernel encode
+    spec = CacheSpec(1, 8, 128, 128, bits, 32)
+    kv = x.repeat(2, 1).reshape(128, 8, 128).to(cuda_device)
+    recs, _ = R.encode_records(kv, kv, spec, 0)
+    pk, pv, sk, sv, _, status = R.gather_records(recs.view(-1), spec, 1)
+    assert status.tolist() == [R.OK]
+    for p, s in ((pk, sk), (pv, sv)):
+        assert np.array_equal(p.cpu().numpy().reshape(-1, packed.shape[-1]), np.tile(packed, (2, 1)))
+        assert np.array_equal(s.cpu().numpy().view(np.uint16).reshape(-1, 4), np.tile(scales.view(np.uint16).reshape(-1, 4), (2, 1)))
