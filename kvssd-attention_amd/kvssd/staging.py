@@ -226,6 +226,16 @@ class RecordStager:
         self.compute_stream = compute_stream
         self.layout = BatchLayout.for_spec(spec, stage_blocks)
         self.slots = [Slot(spec, self.layout, device) for _ in range(slots)]
+        if device.type == "cuda":
+            # the slots' device memory belongs to the stream current here: its
+            # earlier uses there end before the ring's streams write it, and it
+            # is not handed out again before their work on it has ended
+            current = torch.cuda.current_stream(device)
+            for stream in (*self.transfer_streams, compute_stream):
+                stream.wait_stream(current)
+                for slot in self.slots:
+                    slot.raw.record_stream(stream)
+                    slot.batch.record_stream(stream)
         self._record_layout = _native.RecordLayout(
             spec.bits, spec.block_tokens, spec.kv_heads, spec.head_dim, spec.group_size
         )

@@ -306,3 +306,33 @@ def test_store_created_on_gpu_is_byte_identical(cuda_device, tmp_path: Path, bit
     pv, sv, _ = O.quantize_blocks(values[1].float().numpy(), bits, 32, 128)
     ref, _ = O.attention(query.float().numpy(), pk, pv, sk, sv, valid, bits, 32, 1 / math.sqrt(128))
     np.testing.assert_allclose(out.float().cpu().numpy(), ref, atol=ATOL, rtol=RTOL)
+
+
+def test_ring_waits_for_its_memorys_earlier_uses(cuda_device):
+    # the ring's buffers come from memory that the caller's stream still writes (freed, its
+    # last kernel not yet run): the copies of the ring's own streams wait for that
+    from kvssd import records_hip as R
+    from kvssd.staging import HostRecords, RecordStager
+
+    dev = cuda_device
+    spec = CacheSpec(1, 8, 128, 128, 4, 32)
+    gen = torch.Generator(device=dev).manual_seed(3)
+    kv = torch.randn(2, 12 * 128, 8, 128, generator=gen, device=dev).half()
+    query = torch.randn(32, 128, generator=gen, device=dev).half()
+    records, _ = R.encode_records(kv[0], kv[1], spec, 0)
+    pinned = torch.empty(records.shape, dtype=torch.uint8, pin_memory=True)
+    pinned.copy_(records)
+    pk, pv, sk, sv, valid, _ = R.gather_records(records.view(-1), spec, 12)
+    backend = HipAttentionBackend()
+    ref_out, ref_lse = backend.run(query, PackedBatch(pk, pv, sk, sv, valid, 4, 32), 0.1)
+    transfer, compute = torch.cuda.Stream(dev), torch.cuda.Stream(dev)
+    torch.cuda.synchronize()
+    earlier = [torch.empty(4 * spec.record_bytes, dtype=torch.uint8, device=dev) for _ in range(8)]
+    torch.cuda._sleep(20_000_000)
+    for t in earlier:
+        t.fill_(255)
+    del earlier, t
+    stager = RecordStager(spec, dev, 4, backend, transfer, compute)
+    out, lse = stager.run(query, 0.1, 0, list(range(12)), lambda ids, slot: HostRecords(pinned, list(range(12))).spans(ids, spec.record_bytes))
+    torch.testing.assert_close(out, ref_out, atol=1e-4, rtol=1e-3)
+    torch.testing.assert_close(lse, ref_lse, atol=1e-4, rtol=1e-4)
