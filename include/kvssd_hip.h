@@ -194,6 +194,16 @@ int kvssd_hip_gather_records(const kvssd_record_layout* layout, const uint8_t* r
                              int verify_crc, uint8_t* packed_k, uint8_t* packed_v, uint16_t* scales_k,
                              uint16_t* scales_v, int32_t* valid, int32_t* status, void* stream);
 
+/* kvssd_hip_gather_records for the records in rows rows[0 .. n) of the
+ * num_records at `records`; a row outside them gets status 1 and no valid
+ * token.  `records` and `rows` are read where they are: in device memory or in
+ * page-locked host memory, which must stay in place until the launch has run.
+ * Every record is read once where all four arrays are multiples of 16 bytes
+ * per record (and 16-byte aligned), else twice. */
+int kvssd_hip_gather_rows(const kvssd_record_layout* layout, const uint8_t* records, size_t stride, int num_records,
+                          const int32_t* rows, int n, int verify_crc, uint8_t* packed_k, uint8_t* packed_v,
+                          uint16_t* scales_k, uint16_t* scales_v, int32_t* valid, int32_t* status, void* stream);
+
 /* Groupwise quantisation of `rows` rows of `head_dim` values of `dtype`
  * (kvssd_dtype): packed [rows, head_dim*bits/8] (low bits first), fp16 scales
  * [rows, head_dim/group_size].  Bit-exact twin of quantize_tensor

@@ -365,8 +365,17 @@ __attribute__((visibility("default"))) int kvssd_hip_gather_records(
     const kvssd_record_layout* layout, const uint8_t* records, size_t stride, int n, int verify_crc,
     uint8_t* packed_k, uint8_t* packed_v, uint16_t* scales_k, uint16_t* scales_v, int32_t* valid, int32_t* status,
     void* stream) {
-  return launch_gather_records(layout, records, stride, n, verify_crc, packed_k, packed_v, scales_k, scales_v, valid,
-                               status, static_cast<hipStream_t>(stream));
+  return launch_gather_records(layout, records, stride, n, nullptr, n, verify_crc, packed_k, packed_v, scales_k,
+                               scales_v, valid, status, static_cast<hipStream_t>(stream));
+}
+
+__attribute__((visibility("default"))) int kvssd_hip_gather_rows(
+    const kvssd_record_layout* layout, const uint8_t* records, size_t stride, int num_records, const int32_t* rows,
+    int n, int verify_crc, uint8_t* packed_k, uint8_t* packed_v, uint16_t* scales_k, uint16_t* scales_v,
+    int32_t* valid, int32_t* status, void* stream) {
+  if (n > 0 && rows == nullptr) return arg_error("a required buffer pointer is NULL");
+  return launch_gather_records(layout, records, stride, num_records, rows, n, verify_crc, packed_k, packed_v,
+                               scales_k, scales_v, valid, status, static_cast<hipStream_t>(stream));
 }
 
 __attribute__((visibility("default"))) int kvssd_hip_quantize(const void* x, int dtype, int64_t rows, int head_dim,

@@ -90,9 +90,9 @@ int launch_merge_chunks(int rows, int dim, float* acc_out, float* acc_lse, const
                         hipStream_t stream);
 // ---- record codec (records.hip)
 int record_bytes_of(const kvssd_record_layout* layout, size_t* bytes);
-int launch_gather_records(const kvssd_record_layout* layout, const uint8_t* records, size_t stride, int n,
-                          int verify_crc, uint8_t* packed_k, uint8_t* packed_v, uint16_t* scales_k,
-                          uint16_t* scales_v, int32_t* valid, int32_t* status, hipStream_t stream);
+int launch_gather_records(const kvssd_record_layout* layout, const uint8_t* records, size_t stride, int num_records,
+                          const int32_t* rows, int n, int verify_crc, uint8_t* packed_k, uint8_t* packed_v,
+                          uint16_t* scales_k, uint16_t* scales_v, int32_t* valid, int32_t* status, hipStream_t stream);
 int launch_quantize(const void* x, int dtype, int64_t rows, int head_dim, int bits, int group_size, uint8_t* packed,
                     uint16_t* scales, hipStream_t stream);
 int launch_encode_records(const kvssd_record_layout* layout, int dtype, const void* keys, const void* values,

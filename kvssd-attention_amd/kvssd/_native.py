@@ -82,6 +82,7 @@ SIGNATURES = {
     "kvssd_hip_dequantize": (_I, [_VP, _VP, _I64, _I, _I, _I, _VP, _VP]),
     "kvssd_hip_record_bytes": (_I, [ctypes.POINTER(RecordLayout), ctypes.POINTER(_SZ)]),
     "kvssd_hip_gather_records": (_I, [ctypes.POINTER(RecordLayout), _VP, _SZ, _I, _I] + [_VP] * 7),
+    "kvssd_hip_gather_rows": (_I, [ctypes.POINTER(RecordLayout), _VP, _SZ, _I, _VP, _I, _I] + [_VP] * 7),
     "kvssd_hip_quantize": (_I, [_VP, _I, _I64, _I, _I, _I, _VP, _VP, _VP]),
     "kvssd_hip_encode_records": (_I, [ctypes.POINTER(RecordLayout), _I, _VP, _VP, _I64, _I, _I, _VP, _VP, _VP]),
     "kvssd_hip_vllm_sizes": (_I, [_I64, _I, _I, ctypes.POINTER(_SZ), ctypes.POINTER(_SZ)]),

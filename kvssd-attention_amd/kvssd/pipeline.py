@@ -16,7 +16,8 @@ re-planned for MI355X:
   kernel (the reference issues about six torch launches, pipeline.py:147-153).
 * Two resident tiers sit above the SSD: ``load_host_resident`` keeps a layer's
   raw records in page-locked host memory, so a decode of it only streams
-  PCIe; ``load_resident`` keeps the gathered PackedBatch of a layer in HBM
+  PCIe (read by the gather kernel itself, or copied where ``stage_blocks``
+  makes chunks of 8 MiB or more); ``load_resident`` keeps the gathered PackedBatch of a layer in HBM
   (288 GB per MI355X), and a decode of it is a single fused call over a device
   block table with no SSD or PCIe traffic.
 """

@@ -24,6 +24,11 @@ chunk stays in the on-disk record form end to end:
   of microseconds per chunk, while the host-side wait costs nothing when the
   ring is deep enough that it rarely blocks.
 
+A layer kept in page-locked host memory takes no copies at all where its chunks
+would be small: the gather kernel reads the records over PCIe itself, a window of
+the selection per launch, and one fused decode takes the whole window
+(``RecordStager._loop_direct``).
+
 Record statuses of the whole decode collect in one device vector, read back
 once at the end: a bad header or layout raises ValueError and a CRC mismatch
 IOError, with decode_record's messages (src/kvssd/format.py:140-152).
@@ -47,6 +52,13 @@ from .records_hip import gather_records, raise_for_status
 
 SLOTS = 3
 _ALIGN = 256
+# Chunks of at least this many bytes are copied, smaller ones are read by the
+# gather kernel: per 1,024 records of 148 KiB, copies of 4, 16, 32 and 64 records
+# take 5.1, 3.3, 3.0 and 2.7 ms (and, at 4, the host 52 us a chunk for its
+# copy, events and launches), reads by the kernel 2.8 ms whatever the chunk.
+_COPY_CHUNK_BYTES = 8 << 20
+# device bytes of packed arrays a direct decode fills at a time (1.2 ms of PCIe)
+_WINDOW_BYTES = 64 << 20
 
 # (host address, byte offset into the slot's device records, bytes)
 Span = tuple[int, int, int]
@@ -132,6 +144,13 @@ class HostRecords:
 
     def __post_init__(self) -> None:
         self.row_of = {b: i for i, b in enumerate(self.block_ids)}
+        self._device_readable: bool | None = None
+
+    def device_readable(self) -> bool:
+        """Whether a kernel can read the records where they are (page-locked, rows back to back)."""
+        if self._device_readable is None:
+            self._device_readable = self.records.is_contiguous() and self.records.is_pinned()
+        return self._device_readable
 
     def spans(self, ids: Sequence[int], record_bytes: int) -> list[Span]:
         """One span per run of consecutive rows, in the order of ``ids``."""
@@ -148,6 +167,17 @@ class HostRecords:
 
 # fill(ids, slot) puts the raw records of ``ids`` where the returned spans point
 Fill = Callable[[Sequence[int], Slot], list[Span]]
+
+
+class HostFill:
+    """Chunks copied straight from a layer kept in page-locked memory."""
+
+    def __init__(self, host: HostRecords, record_bytes: int):
+        self.host = host
+        self.record_bytes = record_bytes
+
+    def __call__(self, ids: Sequence[int], slot: Slot) -> list[Span]:
+        return self.host.spans(ids, self.record_bytes)
 
 
 class ReadFill:
@@ -242,13 +272,16 @@ class RecordStager:
         self.last_enqueue_seconds = 0.0  # host time the last run spent issuing its chunks
         # record statuses of a run whose check is deferred: (event, host codes, layer, ids)
         self.defer_checks = False
-        self._pending: tuple[torch.cuda.Event, torch.Tensor, int, list[int]] | None = None
+        # (and the host memory the run's kernels read)
+        self._pending: tuple[torch.cuda.Event, torch.Tensor, int, list[int], object] | None = None
+        # direct decodes: the packed arrays of one window, in the compute stream's order
+        self.window_bytes = _WINDOW_BYTES
+        self._window: torch.Tensor | None = None
 
     # ------------------------------------------------------------- fills ---
     def host_fill(self, host: HostRecords) -> Fill:
-        """Chunks copied straight from a layer kept in page-locked memory."""
-        rb = self.spec.record_bytes
-        return lambda ids, slot: host.spans(ids, rb)
+        """Chunks of a layer kept in page-locked memory."""
+        return HostFill(host, self.spec.record_bytes)
 
     def read_fill(self, read: Callable[[Sequence[int], torch.Tensor], Callable[[], None]]) -> "ReadFill":
         """Chunks read into the slot's host memory by ``read(ids, rows)``,
@@ -290,7 +323,7 @@ class RecordStager:
         """Raise for the records of a deferred run (blocks until it finished)."""
         pending, self._pending = self._pending, None
         if pending is not None:
-            event, codes, layer, ids = pending
+            event, codes, layer, ids, _ = pending
             event.synchronize()
             raise_for_status(codes, layer, ids)
 
@@ -312,8 +345,11 @@ class RecordStager:
         with torch.cuda.stream(compute):
             status = torch.empty(len(block_ids), dtype=torch.int32, device=self.device)
             t0 = time.perf_counter()
+            reads = None
             try:
-                if isinstance(self.backend, HipAttentionBackend) and query.dtype in _native.QUERY_DTYPES:
+                if self._direct(query, fill):
+                    acc, reads = self._loop_direct(query, sm_scale, fill.host, block_ids, status)
+                elif isinstance(self.backend, HipAttentionBackend) and query.dtype in _native.QUERY_DTYPES:
                     acc = self._loop_native(query, sm_scale, chunks, fill, status)
                 else:
                     acc = self._loop_generic(query, sm_scale, chunks, fill, status)
@@ -326,7 +362,7 @@ class RecordStager:
             codes.copy_(status, non_blocking=True)
             ready = torch.cuda.Event()
             ready.record(compute)
-        self._pending = (ready, codes, layer, list(block_ids))
+        self._pending = (ready, codes, layer, list(block_ids), reads)
         if not self.defer_checks:
             self.check_pending()
         done = torch.cuda.Event()
@@ -358,19 +394,15 @@ class RecordStager:
         assert acc is not None
         return acc
 
-    def _loop_native(self, query, sm_scale, chunks, fill, status):
-        """The hip backend: every per-chunk launch goes straight to the C ABI
-        with descriptors and pointers prepared once per decode, so the host
-        spends a few ctypes calls per chunk and keeps ahead of the copies."""
-        spec, sb, compute = self.spec, self.stage_blocks, self.compute_stream
-        lib = _native.load()
-        q = query.contiguous()
+    def _describe(self, q: torch.Tensor, sm_scale: float, counts: set[int], kernel: int | None = None) -> tuple[dict, int]:
+        """Decode descriptors for batches of each of ``counts`` blocks, and the largest workspace."""
+        spec = self.spec
         # the reference's argument checks, once (every chunk has the same shape)
         PackedBatch(*self.layout.views(self.slots[0].batch, spec, 1), spec.bits, spec.group_size).validate(q)
         qh, dim = q.shape
         descs: dict[int, _native.DecodeDesc] = {}
         need = 1
-        for n in {len(c) for c in chunks}:
+        for n in counts:
             d = _native.DecodeDesc(
                 query_heads=qh,
                 kv_heads=spec.kv_heads,
@@ -381,13 +413,94 @@ class RecordStager:
                 group_size=spec.group_size,
                 query_dtype=_native.QUERY_DTYPES[q.dtype],
                 num_selected=0,
-                kernel=self.backend.kernel,
+                kernel=self.backend.kernel if kernel is None else kernel,
                 sm_scale=float(sm_scale),
             )
             nbytes = ctypes.c_size_t(0)
-            _native.check(lib.kvssd_hip_decode_workspace_bytes(ctypes.byref(d), ctypes.byref(nbytes)), "workspace")
+            _native.check(
+                _native.load().kvssd_hip_decode_workspace_bytes(ctypes.byref(d), ctypes.byref(nbytes)), "workspace"
+            )
             need = max(need, int(nbytes.value))
             descs[n] = d
+        return descs, need
+
+    def _direct(self, query: torch.Tensor, fill: Fill) -> bool:
+        """Whether the gather kernel reads the records from host memory itself:
+        chunks too small for copies at PCIe's rate, and a layout that the
+        gather reads once (all four arrays whole 16-byte chunks)."""
+        return (
+            isinstance(fill, HostFill)
+            and isinstance(self.backend, HipAttentionBackend)
+            and query.dtype in _native.QUERY_DTYPES
+            and self.stage_blocks * self.spec.record_bytes < _COPY_CHUNK_BYTES
+            and self.layout.packed % 16 == 0
+            and self.layout.scales % 16 == 0
+            and fill.host.device_readable()
+        )
+
+    def _loop_direct(self, query, sm_scale, host, block_ids, status):
+        """Gather each window of the selection straight out of page-locked host
+        memory and decode it in one call: on one stream and with no copies, two
+        launches a window (the gather, at PCIe's rate, takes ~100 times the
+        decode's time, so overlapping them would gain nothing).  Returns the
+        result and the host memory that the launches read."""
+        spec = self.spec
+        lib = _native.load()
+        q = query.contiguous()
+        total = len(block_ids)
+        per_block = 2 * (self.layout.packed + self.layout.scales)
+        windows = -(-total // max(1, self.window_bytes // per_block))
+        size = -(-total // windows)
+        counts = [min(size, total - i) for i in range(0, total, size)]
+        # a window takes the kernel that a chunk of it would (AUTO's choice for few
+        # blocks): its output error is the smaller one (16K tokens, 8 kv heads, fp32:
+        # 6.4e-5 against 9.1e-5)
+        chunk, _ = self._describe(q, sm_scale, {min(self.stage_blocks, total)})
+        kernel = ctypes.c_int(0)
+        rc = lib.kvssd_hip_decode_kernel(ctypes.byref(next(iter(chunk.values()))), ctypes.byref(kernel))
+        _native.check(rc, "kvssd_hip_decode_kernel")
+        descs, need = self._describe(q, sm_scale, set(counts), kernel.value)
+        L = BatchLayout.for_spec(spec, size)
+        if self._window is None or self._window.numel() < L.total:
+            self._window = torch.empty(L.total, dtype=torch.uint8, device=self.device)
+        b = self._window.data_ptr()
+        kp, vp, ks, vs, va = b + L.off_kp, b + L.off_vp, b + L.off_ks, b + L.off_vs, b + L.off_valid
+        qh, dim = q.shape
+        work = torch.empty(need, dtype=torch.uint8, device=self.device)
+        out = torch.empty((min(len(counts), 2), qh, dim), dtype=torch.float32, device=self.device)
+        lse = torch.empty((min(len(counts), 2), qh), dtype=torch.float32, device=self.device)
+        # the records' rows, read by the kernel where they are
+        rows = torch.empty(total, dtype=torch.int32, pin_memory=True)
+        rows.numpy()[:] = [host.row_of[i] for i in block_ids]
+        cs = _native.stream_handle(self.compute_stream)
+        lay = ctypes.byref(self._record_layout)
+        first = 0
+        for i, n in enumerate(counts):
+            rc = lib.kvssd_hip_gather_rows(
+                lay, host.records.data_ptr(), spec.record_bytes, host.records.shape[0], rows.data_ptr() + 4 * first, n, 1,
+                kp, vp, ks, vs, va, status.data_ptr() + 4 * first, cs,
+            )
+            _native.check(rc, "kvssd_hip_gather_rows")
+            o, l = out[min(i, 1)], lse[min(i, 1)]
+            rc = lib.kvssd_hip_fused_decode(
+                ctypes.byref(descs[n]), q.data_ptr(), kp, vp, ks, vs, va, None, o.data_ptr(), l.data_ptr(),
+                work.data_ptr(), need, cs,
+            )
+            _native.check(rc, "kvssd_hip_fused_decode")
+            if i:
+                self.backend.merge_chunks(out[0], lse[0], o, l)
+            first += n
+        return (out[0], lse[0]), (rows, host)
+
+    def _loop_native(self, query, sm_scale, chunks, fill, status):
+        """The hip backend: every per-chunk launch goes straight to the C ABI
+        with descriptors and pointers prepared once per decode, so the host
+        spends a few ctypes calls per chunk and keeps ahead of the copies."""
+        spec, sb, compute = self.spec, self.stage_blocks, self.compute_stream
+        lib = _native.load()
+        q = query.contiguous()
+        qh, dim = q.shape
+        descs, need = self._describe(q, sm_scale, {len(c) for c in chunks})
         work = torch.empty(need, dtype=torch.uint8, device=self.device)
         acc_out = torch.empty((qh, dim), dtype=torch.float32, device=self.device)
         acc_lse = torch.empty(qh, dtype=torch.float32, device=self.device)

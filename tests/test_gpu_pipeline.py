@@ -308,6 +308,55 @@ def test_store_created_on_gpu_is_byte_identical(cuda_device, tmp_path: Path, bit
     np.testing.assert_allclose(out.float().cpu().numpy(), ref, atol=ATOL, rtol=RTOL)
 
 
+@pytest.mark.parametrize("head_dim", [128, 40])
+def test_host_resident_direct_windows(cuda_device, head_dim: int):
+    # records read by the gather kernel out of page-locked memory: scattered rows, one and
+    # several windows of the selection, a whole-chunk layout (head_dim 40 is not one, and takes
+    # the copies), against one decode of the same records in HBM; a bad record still raises
+    from kvssd import records_hip as R
+    from kvssd.backends import PackedBatch
+    from kvssd.format import CacheSpec
+    from kvssd.staging import HostRecords, RecordStager
+
+    dev = cuda_device
+    spec = CacheSpec(1, 2, head_dim, 33 if head_dim == 40 else 32, 4, 20 if head_dim == 40 else 32)
+    gen = torch.Generator(device=dev).manual_seed(head_dim)
+    kv = torch.randn(2, 20 * spec.block_tokens - 5, 2, head_dim, generator=gen, device=dev).half()
+    query = torch.randn(8, head_dim, generator=gen, device=dev).half()
+    records, _ = R.encode_records(kv[0], kv[1], spec, 0)
+    pinned = torch.empty(records.shape, dtype=torch.uint8, pin_memory=True)
+    pinned.copy_(records)
+    host = HostRecords(pinned, list(range(100, 120)))
+    backend = HipAttentionBackend()
+    stager = RecordStager(spec, dev, 4, backend, torch.cuda.Stream(dev), torch.cuda.Stream(dev))
+    pk, pv, sk, sv, valid, _ = R.gather_records(records.view(-1), spec, 20)
+    for rows in ([0], [7, 3, 4, 19, 0], list(range(20)), list(range(19, -1, -2))):
+        ids = [100 + r for r in rows]
+        batch = PackedBatch(pk, pv, sk, sv, valid, 4, spec.group_size)
+        ref_out, ref_lse = backend.run(query, batch, 0.2, block_table=rows)
+        for window in (1, 3 * 2 * 32 * 2 * (64 + 8), 64 << 20):
+            stager.window_bytes = window
+            out, lse = stager.run(query, 0.2, 0, ids, stager.host_fill(host))
+            torch.testing.assert_close(out, ref_out, atol=1e-4, rtol=1e-3)
+            torch.testing.assert_close(lse, ref_lse, atol=1e-4, rtol=1e-4)
+    pinned[7, 52 + 100] ^= 4
+    with pytest.raises(IOError, match="block=107"):
+        stager.run(query, 0.2, 0, [101, 107, 119], stager.host_fill(host))
+    # a row outside the records is refused by the kernel, unread
+    import ctypes
+
+    from kvssd import _native
+
+    out = R.gather_records(records.view(-1), spec, 2)
+    rows_dev = torch.tensor([20, 19], dtype=torch.int32, device=dev)
+    lay = _native.RecordLayout(4, spec.block_tokens, 2, head_dim, spec.group_size)
+    rc = _native.load().kvssd_hip_gather_rows(
+        ctypes.byref(lay), records.data_ptr(), spec.record_bytes, 20, rows_dev.data_ptr(), 2, 1,
+        *[t.data_ptr() for t in out], _native.stream_handle(torch.cuda.current_stream()),
+    )
+    assert rc == 0 and out[5].tolist() == [R.BAD_HEADER, R.OK] and out[4].tolist() == [0, valid[19].item()]
+
+
 def test_ring_waits_for_its_memorys_earlier_uses(cuda_device):
     # the ring's buffers come from memory that the caller's stream still writes (freed, its
     # last kernel not yet run): the copies of the ring's own streams wait for that
