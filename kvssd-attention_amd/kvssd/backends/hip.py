@@ -130,7 +130,9 @@ class HipAttentionBackend:
         query's dtype: then the merge stores it in that dtype, rounded to
         nearest even -- the values ``out.to(query.dtype)`` would give, without
         the extra cast kernel.  ``lse`` is fp32 either way."""
-        return self.prepare(query, batch, sm_scale, block_table, out_dtype)(query)
+        # one call needs one row of output: the block of rows a kept decode
+        # hands out costs the host ~45 us to make and take apart
+        return PreparedDecode(self, query, batch, sm_scale, block_table, out_dtype, rows=1)(query)
 
     def prepare(
         self,
@@ -229,7 +231,9 @@ class PreparedDecode:
     _MAX_STREAMS = 8
     _ROWS = 64
 
-    def __init__(self, backend: HipAttentionBackend, query, batch, sm_scale, block_table, out_dtype):
+    def __init__(
+        self, backend: HipAttentionBackend, query, batch, sm_scale, block_table, out_dtype, rows: int = _ROWS
+    ):
         if out_dtype is not None and out_dtype not in (torch.float32, query.dtype):
             raise ValueError(f"out_dtype must be torch.float32 or the query's dtype {query.dtype}, got {out_dtype}")
         typed = out_dtype is not None and out_dtype != torch.float32
@@ -279,6 +283,7 @@ class PreparedDecode:
         self._qshape = tuple(query.shape)
         self._qsize = torch.Size(self._qshape)
         self._qdtype = query.dtype
+        self._rows = rows
         self._out_shape = (query.shape[0], query.shape[1])
         self._out_dtype = query.dtype if typed else torch.float32
         # per stream: [workspace pointer, workspace bytes, out row pointers,
@@ -316,8 +321,8 @@ class PreparedDecode:
             work = torch.empty((max(self._need, 1),), dtype=torch.uint8, device=self._device)
         else:
             work = old[7]
-        outs = torch.empty((self._ROWS, *self._out_shape), dtype=self._out_dtype, device=self._device).unbind(0)
-        lses = torch.empty((self._ROWS, self._out_shape[0]), dtype=torch.float32, device=self._device).unbind(0)
+        outs = torch.empty((self._rows, *self._out_shape), dtype=self._out_dtype, device=self._device).unbind(0)
+        lses = torch.empty((self._rows, self._out_shape[0]), dtype=torch.float32, device=self._device).unbind(0)
         slot = [
             work.data_ptr(), work.numel(), [t.data_ptr() for t in outs], [t.data_ptr() for t in lses], 0, outs, lses,
             work,
@@ -328,7 +333,7 @@ class PreparedDecode:
     def _launch(self, q: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         handle = current_stream_handle(self._index)
         slot = self._slots.get(handle)
-        if slot is None or slot[4] == self._ROWS:
+        if slot is None or slot[4] == self._rows:
             slot = self._slot(handle, slot)
         i = slot[4]
         slot[4] = i + 1
