@@ -234,41 +234,44 @@ struct GroupWords {
 // * 32-bit values: q = x r is off by less than 2^-19, so that its nearest
 //   integer is right unless q lies within 2^-18 of some k + 0.5; then, and for
 //   scales whose reciprocal is subnormal or zero, the division itself.
+// Only the division's form needs the clamp, for NaN: a NaN shows in the sums.
 template <typename T, int BITS>
 __device__ __forceinline__ uint32_t code_word(const float (&x)[32 / BITS], float s32) {
-  constexpr int kCodes = 32 / BITS;
+  constexpr int kCodes = 32 / BITS, n = kCodes / 2;
   constexpr float mid = static_cast<float>(1 << (BITS - 1));
-  float c[kCodes];
+  constexpr float radix = static_cast<float>(1 << BITS);
+  float half[2];  // 16 bits at a time as an exact float sum
   bool done = false;
   if (s32 < 0x1p120f) {
     const float r0 = __builtin_amdgcn_rcpf(s32);
     const float r = __builtin_fmaf(__builtin_fmaf(-s32, r0, 1.0f), r0, r0);
     float off = 0.0f;
 #pragma unroll
-    for (int i = 0; i < kCodes; ++i) {
-      float q = x[i] * r;
-      if constexpr (sizeof(T) == 2) q = __builtin_fmaf(__builtin_fmaf(-q, s32, x[i]), r, q);
-      const float n = rintf(q);
-      if constexpr (sizeof(T) != 2) off = fmaxf(off, fabsf(q - n));
-      c[i] = fminf(fmaxf(n, -mid), mid - 1.0f);
+    for (int k = 0; k < 2; ++k) {
+      float t = 0.0f;
+#pragma unroll
+      for (int i = n - 1; i >= 0; --i) {
+        const float v = x[k * n + i];
+        float q = v * r;
+        if constexpr (sizeof(T) == 2) q = __builtin_fmaf(__builtin_fmaf(-q, s32, v), r, q);
+        const float c = rintf(q);  // within +-(mid - 1), or NaN, and then so is the sum
+        if constexpr (sizeof(T) != 2) off = fmaxf(off, fabsf(q - c));
+        t = i == n - 1 ? c : __builtin_fmaf(t, radix, c);
+      }
+      half[k] = t + static_cast<float>(BITS == 4 ? 0x8888 : 0xAAAA);  // mid for every code
     }
-    done = sizeof(T) == 2 || off < 0.5f - 0x1p-18f;
+    done = half[0] == half[0] && half[1] == half[1] && (sizeof(T) == 2 || off < 0.5f - 0x1p-18f);
   }
   if (!done) {
 #pragma unroll
-    for (int i = 0; i < kCodes; ++i) c[i] = fminf(fmaxf(rintf(x[i] / s32), -mid), mid - 1.0f);
-  }
-  // 16 bits at a time as an exact float sum
-  uint32_t half[2];
+    for (int k = 0; k < 2; ++k) {
+      half[k] = 0.0f;
 #pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    constexpr int n = kCodes / 2;
-    float t = c[k * n + n - 1] + mid;
-#pragma unroll
-    for (int i = n - 2; i >= 0; --i) t = __builtin_fmaf(t, static_cast<float>(1 << BITS), c[k * n + i] + mid);
-    half[k] = static_cast<uint32_t>(t);
+      for (int i = n - 1; i >= 0; --i)
+        half[k] = __builtin_fmaf(half[k], radix, fminf(fmaxf(rintf(x[k * n + i] / s32), -mid), mid - 1.0f) + mid);
+    }
   }
-  return half[0] | (half[1] << 16);
+  return static_cast<uint32_t>(half[0]) | (static_cast<uint32_t>(half[1]) << 16);
 }
 
 // max(amax, 1e-8) / (mid - 1), IEEE
@@ -446,7 +449,7 @@ __global__ __launch_bounds__(kCrcThreads) void encode_header_kernel(EncodeParams
 // in LDS; after a barrier they are stored and take a CRC of their own, moved
 // before the codes' by one multiply, so the payload is never read back.
 // Measured (1,024 records of 8 kv heads, head_dim 128, bfloat16, 688 MB moved):
-// a lane a group, reading 64 bytes of its own, and IEEE divisions 222 us, 178
+// a lane a group, reading 64 bytes of its own, and IEEE divisions 222 us, 174
 // us in this form.
 struct FusedPlan {
   int rows_s, rows_c;  // rows of scale / code chunks

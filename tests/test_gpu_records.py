@@ -278,3 +278,27 @@ def test_quantize_around_ties(cuda_device, bits, dtype):
     for p, s in ((pk, sk), (pv, sv)):
         assert np.array_equal(p.cpu().numpy().reshape(-1, packed.shape[-1]), np.tile(packed, (2, 1)))
         assert np.array_equal(s.cpu().numpy().view(np.uint16).reshape(-1, 4), np.tile(scales.view(np.uint16).reshape(-1, 4), (2, 1)))
+
+
+@pytest.mark.parametrize("bits", [2, 4])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_quantize_nan_and_infinity(cuda_device, bits, dtype):
+    # a NaN takes code 0 and leaves its group's scale alone; a group with an infinity has an
+    # infinite scale, so finite values take the middle code and the infinity (inf / inf) code 0;
+    # the register form (group 32) as the element-wise one (the same values in a shifted source)
+    gen = torch.Generator().manual_seed(17)
+    x = torch.randn(64, 128, generator=gen)
+    x[3, 5] = x[9, 64] = x[9, 71] = float("nan")
+    x[12, 0], x[20, 127], x[31, 40] = float("inf"), float("-inf"), float("inf")
+    x[31, 41] = float("nan")
+    x[40, 32:64] = float("nan")
+    x = x.to(dtype).to(cuda_device)
+    buf = torch.empty(64 * 128 + 1, dtype=dtype, device=cuda_device)
+    shifted = buf[1:].view(64, 128)
+    shifted.copy_(x)
+    a, b = R.quantize(x, bits, 32), R.quantize(shifted, bits, 32)
+    assert torch.equal(a.packed, b.packed) and torch.equal(a.scales.view(torch.int16), b.scales.view(torch.int16))
+    per = 8 // bits
+    codes = torch.stack([(a.packed >> (bits * i)) & ((1 << bits) - 1) for i in range(per)], -1).reshape(64, 128).cpu()
+    assert codes[3, 5] == 0 and codes[12, 0] == 0 and codes[20, 127] == 0 and (codes[40, 32:64] == 0).all()
+    assert (codes[12, 1:32] == 1 << (bits - 1)).all() and torch.isinf(a.scales[12, 0]) and torch.isfinite(a.scales[3]).all()
