@@ -254,12 +254,18 @@ struct ChunkLds {
   uint32_t seg[kCrcThreads / 64];
 };
 
+// by a workgroup of kCrcThreads / PARTS threads
+template <int PARTS = 1>
 __device__ __forceinline__ void load_chunk_tables(ChunkLds& l, const BitMatrices& m = kBitMatrices) {
+  constexpr int threads = kCrcThreads / PARTS;
   const u32x4* src = reinterpret_cast<const u32x4*>(&m);
   u32x4* dst = &l.data[0][0][0];  // data then carry: 1024 + 64 entries
-  const u32x4 v = src[threadIdx.x];
+  u32x4 v[PARTS];
+#pragma unroll
+  for (int i = 0; i < PARTS; ++i) v[i] = src[threadIdx.x + i * threads];
   if (threadIdx.x < 64) dst[kCrcThreads + threadIdx.x] = src[kCrcThreads + threadIdx.x];
-  dst[threadIdx.x] = v;
+#pragma unroll
+  for (int i = 0; i < PARTS; ++i) dst[threadIdx.x + i * threads] = v[i];
 }
 
 // 16 bytes at a 4-byte aligned address
@@ -338,22 +344,34 @@ __device__ __forceinline__ int64_t chunk_offset(const ChunkPlan& c, int j) {
   return (static_cast<int64_t>(j) * kCrcThreads + threadIdx.x) * kChunkBytes - c.pad;
 }
 
-// Fold the column states h of crc_group over the workgroup: a column ends with
-// its half-1 chunk (pos[t] = the shift of piece t to the end).  The raw register
+// Fold the column states h of crc_group over the workgroup, thread t holding
+// those of threads t, t + 1024 / PARTS, ... of 1024: a column ends with its
+// half-1 chunk (pos[t] = the shift of piece t to the end).  The raw register
 // value of the whole message is returned in every thread.
-__device__ uint32_t fold_columns(ChunkLds& l, const uint32_t* pos, uint32_t h) {
+template <int PARTS>
+__device__ __forceinline__ uint32_t fold_columns(ChunkLds& l, const uint32_t* pos, const uint32_t (&h)[PARTS]) {
+  constexpr int threads = kCrcThreads / PARTS;
   const int tid = threadIdx.x;
-  h |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(h), 32, 64));
-  uint32_t v = gf_mul_dev(pos[tid | 32], h);
+  uint32_t v = 0;
+#pragma unroll
+  for (int i = 0; i < PARTS; ++i) {
+    const uint32_t column = h[i] | static_cast<uint32_t>(__shfl_xor(static_cast<int>(h[i]), 32, 64));
+    v ^= gf_mul_dev(pos[(tid + i * threads) | 32], column);
+  }
 #pragma unroll
   for (int off = 16; off > 0; off >>= 1) v ^= static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), off, 64));
   if ((tid & 63) == 0) l.seg[tid >> 6] = v;
   __syncthreads();
   uint32_t raw = 0;
 #pragma unroll
-  for (int w = 0; w < kCrcThreads / 64; ++w) raw ^= l.seg[w];
+  for (int w = 0; w < threads / 64; ++w) raw ^= l.seg[w];
   __syncthreads();  // seg may be reused by the caller
   return raw;
+}
+
+__device__ __forceinline__ uint32_t fold_columns(ChunkLds& l, const uint32_t* pos, uint32_t h) {
+  const uint32_t one[1] = {h};
+  return fold_columns<1>(l, pos, one);
 }
 
 // Fold one value per thread, thread t's piece followed by the pieces of threads

@@ -449,13 +449,14 @@ __global__ __launch_bounds__(kCrcThreads) void encode_header_kernel(EncodeParams
 // in LDS; after a barrier they are stored and take a CRC of their own, moved
 // before the codes' by one multiply, so the payload is never read back.
 // Measured (1,024 records of 8 kv heads, head_dim 128, bfloat16, 688 MB moved):
-// a lane a group, reading 64 bytes of its own, and IEEE divisions 222 us, 174
+// a lane a group, reading 64 bytes of its own, and IEEE divisions 222 us, 166
 // us in this form.
 struct FusedPlan {
   int rows_s, rows_c;  // rows of scale / code chunks
   uint32_t x_codes;    // x^(8 * code bytes) mod P
 };
 
+constexpr int kComputeUnits = 256;
 constexpr int kMaxScaleRows = kGroupRows;  // scale region <= 64 KiB of LDS, one group of rows
 
 // largest of v over the BITS lanes (4 or 2) that share a group
@@ -467,8 +468,11 @@ __device__ __forceinline__ float group_max(float v) {
   return v;
 }
 
-template <typename T, int BITS>
-__global__ __launch_bounds__(kCrcThreads) void encode_fused_kernel(EncodeParams p, ChunkPlan c, FusedPlan f) {
+// PARTS: the workgroup has 1024 / PARTS threads, each taking the parts of PARTS
+// in turn.
+template <typename T, int BITS, int PARTS>
+__global__ __launch_bounds__(kCrcThreads / PARTS) void encode_fused_kernel(EncodeParams p, ChunkPlan c, FusedPlan f) {
+  constexpr int kThreads = kCrcThreads / PARTS;
   __shared__ ChunkLds lds;
   extern __shared__ __attribute__((aligned(16))) uint16_t scales[];  // the record's scale region
   constexpr int kVals = 32 / BITS;                                   // values of a word of codes
@@ -486,10 +490,12 @@ __global__ __launch_bounds__(kCrcThreads) void encode_fused_kernel(EncodeParams 
   const int64_t block = static_cast<int64_t>(L.block_tokens) * L.kv_heads * L.head_dim;
   const int64_t left = p.tokens * L.kv_heads * L.head_dim - r * block;
   // the values of runs u0 .. u0 + kAhead - 1 of code row k's piece
-  auto piece_of = [&](int k) { return (static_cast<int64_t>(k) * kCrcThreads + (tid & ~63)) * kChunkBytes; };
-  auto load_runs = [&](int k, int u0, uint32_t (&raw)[kAhead][kRaw]) {
+  auto piece_of = [&](int k, int part) {
+    return (static_cast<int64_t>(k) * kCrcThreads + part * kThreads + (tid & ~63)) * kChunkBytes;
+  };
+  auto load_runs = [&](int k, int part, int u0, uint32_t (&raw)[kAhead][kRaw]) {
     // codes of keys or of values (arrays are whole pieces)
-    const int64_t piece = piece_of(k);
+    const int64_t piece = piece_of(k, part);
     const bool is_v = piece >= array;
     const T* base = static_cast<const T*>(is_v ? p.values : p.keys) + r * block;
     const int64_t at = (is_v ? piece - array : piece) * (8 / BITS) + lane * kVals;  // of the block's values
@@ -503,71 +509,81 @@ __global__ __launch_bounds__(kCrcThreads) void encode_fused_kernel(EncodeParams 
     }
   };
   uint32_t next[kAhead][kRaw];
-  load_runs(0, 0, next);
-  load_chunk_tables(lds, kWordMatrices);
+  load_runs(0, 0, 0, next);
+  load_chunk_tables<PARTS>(lds, kWordMatrices);
   __syncthreads();  // the CRC matrices are in LDS
-  uint32_t h = 0;
+  uint32_t codes[PARTS], sums[PARTS];  // column states of the codes, of the scales
   const int lead = (kGroupRows - f.rows_c % kGroupRows) % kGroupRows;  // zero rows of the first group
-  for (int k0 = -lead; k0 < f.rows_c; k0 += kGroupRows) {
-    f32x16 acc = crc_begin(lds, h);
 #pragma unroll 1
-    for (int j = k0 < 0 ? -k0 : 0; j < kGroupRows; ++j) {
-      const int k = k0 + j;
-      const int64_t piece = piece_of(k);
-      u32x4 words;
+  for (int part = 0; part < PARTS; ++part) {
+    uint32_t h = 0;
+    for (int k0 = -lead; k0 < f.rows_c; k0 += kGroupRows) {
+      f32x16 acc = crc_begin(lds, h);
+#pragma unroll 1
+      for (int j = k0 < 0 ? -k0 : 0; j < kGroupRows; ++j) {
+        const int k = k0 + j;
+        const int64_t piece = piece_of(k, part);
+        u32x4 words;
 #pragma unroll
-      for (int u0 = 0; u0 < 4; u0 += kAhead) {
-        uint32_t raw[kAhead][kRaw];
-        __builtin_memcpy(raw, next, sizeof(raw));
-        // the next runs' loads are in flight while these are quantised
-        if (u0 + kAhead < 4) load_runs(k, u0 + kAhead, next);
-        else if (k + 1 < f.rows_c) load_runs(k + 1, 0, next);
-        __builtin_amdgcn_sched_barrier(0);
+        for (int u0 = 0; u0 < 4; u0 += kAhead) {
+          uint32_t raw[kAhead][kRaw];
+          __builtin_memcpy(raw, next, sizeof(raw));
+          // the next runs' loads are in flight while these are quantised
+          if (u0 + kAhead < 4) load_runs(k, part, u0 + kAhead, next);
+          else if (k + 1 < f.rows_c) load_runs(k + 1, part, 0, next);
+          else if (part + 1 < PARTS) load_runs(0, part + 1, 0, next);
+          __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int a = 0; a < kAhead; ++a) {
-          const int u = u0 + a;
-          T v[kVals];
-          __builtin_memcpy(v, raw[a], sizeof(v));
-          float x[kVals], amax = 0.0f;
+          for (int a = 0; a < kAhead; ++a) {
+            const int u = u0 + a;
+            T v[kVals];
+            __builtin_memcpy(v, raw[a], sizeof(v));
+            float x[kVals], amax = 0.0f;
 #pragma unroll
-          for (int i = 0; i < kVals; ++i) {
-            x[i] = to_f32(v[i]);
-            amax = fmaxf(amax, fabsf(x[i]));
+            for (int i = 0; i < kVals; ++i) {
+              x[i] = to_f32(v[i]);
+              amax = fmaxf(amax, fabsf(x[i]));
+            }
+            const float s32 = group_scale<BITS>(group_max<BITS>(amax));
+            const uint32_t word = code_word<T, BITS>(x, s32);
+            words[u] = word;
+            if ((lane & (BITS - 1)) == 0)
+              scales[piece / (4 * BITS) + u * (64 / BITS) + lane / BITS] =
+                  __builtin_bit_cast(uint16_t, static_cast<_Float16>(s32));
+            __builtin_memcpy(__builtin_assume_aligned(pay + code0 + piece + u * kRunBytes + 4 * lane, 4), &word, 4);
+            __builtin_amdgcn_sched_barrier(0);  // (runs quantised side by side would not fit the registers)
           }
-          const float s32 = group_scale<BITS>(group_max<BITS>(amax));
-          const uint32_t word = code_word<T, BITS>(x, s32);
-          words[u] = word;
-          if ((lane & (BITS - 1)) == 0)
-            scales[piece / (4 * BITS) + u * (64 / BITS) + lane / BITS] =
-                __builtin_bit_cast(uint16_t, static_cast<_Float16>(s32));
-          __builtin_memcpy(__builtin_assume_aligned(pay + code0 + piece + u * kRunBytes + 4 * lane, 4), &word, 4);
-          __builtin_amdgcn_sched_barrier(0);  // (runs quantised side by side would not fit the registers)
         }
+        acc = crc_row(lds, acc, j, words);
       }
-      acc = crc_row(lds, acc, j, words);
+      h = crc_end(acc);
     }
-    h = crc_end(acc);
+    if (part == 0) codes[0] = h;
+    else codes[PARTS - 1] = h;
   }
   __syncthreads();  // every scale is in LDS
-  u32x4 v[kGroupRows];
 #pragma unroll
-  for (int j = 0; j < kGroupRows; ++j) {
-    v[j] = u32x4{0u, 0u, 0u, 0u};
-    const int row = j + f.rows_s - kGroupRows;
-    if (row >= 0) {
-      const int64_t piece = (static_cast<int64_t>(row) * kCrcThreads + (tid & ~63)) * kChunkBytes;
+  for (int part = 0; part < PARTS; ++part) {
+    u32x4 v[kGroupRows];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const uint32_t word = reinterpret_cast<const uint32_t*>(scales)[piece / 4 + u * 64 + lane];
-        __builtin_memcpy(__builtin_assume_aligned(pay + piece + u * kRunBytes + 4 * lane, 4), &word, 4);
-        v[j][u] = word;
+    for (int j = 0; j < kGroupRows; ++j) {
+      v[j] = u32x4{0u, 0u, 0u, 0u};
+      const int row = j + f.rows_s - kGroupRows;
+      if (row >= 0) {
+        const int64_t piece = piece_of(row, part);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const uint32_t word = reinterpret_cast<const uint32_t*>(scales)[piece / 4 + u * 64 + lane];
+          __builtin_memcpy(__builtin_assume_aligned(pay + piece + u * kRunBytes + 4 * lane, 4), &word, 4);
+          v[j][u] = word;
+        }
       }
     }
+    sums[part] = crc_group(lds, 0u, v, kGroupRows - f.rows_s);
   }
-  const uint32_t hs = crc_group(lds, 0u, v, kGroupRows - f.rows_s);
   // the scales come before the codes in the message
-  const uint32_t raw_s = fold_columns(lds, kPosTables.word, hs);
-  const uint32_t raw_c = fold_columns(lds, kPosTables.word, h);
+  const uint32_t raw_s = fold_columns<PARTS>(lds, kPosTables.word, sums);
+  const uint32_t raw_c = fold_columns<PARTS>(lds, kPosTables.word, codes);
   const uint32_t crc = crc_from_raw(c.x_len, gf_mul_dev(f.x_codes, raw_s) ^ raw_c);
   const int64_t start = static_cast<int64_t>(r) * L.block_tokens;
   const int64_t valid = p.tokens - start < L.block_tokens ? p.tokens - start : L.block_tokens;
@@ -590,7 +606,7 @@ __global__ __launch_bounds__(kCrcThreads) void encode_fused_kernel(EncodeParams 
     }
     reinterpret_cast<uint32_t*>(rec)[tid] = v;
   }
-  for (int64_t i = kHeaderBytes + L.payload_bytes() + tid; i < L.record_bytes(); i += kCrcThreads) rec[i] = 0;
+  for (int64_t i = kHeaderBytes + L.payload_bytes() + tid; i < L.record_bytes(); i += kThreads) rec[i] = 0;
   if (tid == 0) p.crcs[r] = crc;
 }
 
@@ -643,14 +659,25 @@ void launch_quantize_t(const void* x, int64_t groups, int group_size, int bits, 
   }
 }
 
-template <typename T>
-void launch_fused_t(const EncodeParams& p, const ChunkPlan& c, const FusedPlan& f, hipStream_t s) {
+template <typename T, int PARTS>
+void launch_fused_parts(const EncodeParams& p, const ChunkPlan& c, const FusedPlan& f, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(p.n));
   const size_t scale_lds = static_cast<size_t>(2 * p.lay.scale_bytes());
   if (p.lay.bits == 4)
-    hipLaunchKernelGGL((encode_fused_kernel<T, 4>), grid, dim3(kCrcThreads), scale_lds, s, p, c, f);
+    hipLaunchKernelGGL((encode_fused_kernel<T, 4, PARTS>), grid, dim3(kCrcThreads / PARTS), scale_lds, s, p, c, f);
   else
-    hipLaunchKernelGGL((encode_fused_kernel<T, 2>), grid, dim3(kCrcThreads), scale_lds, s, p, c, f);
+    hipLaunchKernelGGL((encode_fused_kernel<T, 2, PARTS>), grid, dim3(kCrcThreads / PARTS), scale_lds, s, p, c, f);
+}
+
+// Past one record per CU, workgroups of 512 threads: their registers let two
+// share a CU, and one's start and end pass under the other's work (128-token
+// records of 8 kv heads: 257 of them 71 -> 66 us a call, 400 79 -> 74, 1,024
+// 174 -> 170).  Up to there 1024 threads finish a record sooner (256: 42 us
+// against 47, 16: 33 against 37).
+template <typename T>
+void launch_fused_t(const EncodeParams& p, const ChunkPlan& c, const FusedPlan& f, hipStream_t s) {
+  if (p.n > kComputeUnits) launch_fused_parts<T, 2>(p, c, f, s);
+  else launch_fused_parts<T, 1>(p, c, f, s);
 }
 
 template <typename T>

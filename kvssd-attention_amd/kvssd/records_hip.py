@@ -176,4 +176,4 @@ def encode_records(
         _stream(),
     )
     _native.check(rc, "kvssd_hip_encode_records")
-    return records, crcs.to(torch.int64) & 0xFFFFFFFF
+    return records, crcs.view(torch.uint32).to(torch.int64)

@@ -302,3 +302,24 @@ def test_quantize_nan_and_infinity(cuda_device, bits, dtype):
     codes = torch.stack([(a.packed >> (bits * i)) & ((1 << bits) - 1) for i in range(per)], -1).reshape(64, 128).cpu()
     assert codes[3, 5] == 0 and codes[12, 0] == 0 and codes[20, 127] == 0 and (codes[40, 32:64] == 0).all()
     assert (codes[12, 1:32] == 1 << (bits - 1)).all() and torch.isinf(a.scales[12, 0]) and torch.isfinite(a.scales[3]).all()
+
+
+@pytest.mark.parametrize("bits", [2, 4])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_encode_more_records_than_compute_units(cuda_device, bits, dtype):
+    # past 256 records the workgroups are of 512 threads; the same bytes and CRC values as the
+    # same blocks in smaller calls (which other tests hold to the oracle's), for one and several
+    # rows of scales, the last record partly filled
+    for kvh in (8, 16):
+        spec = CacheSpec(1, kvh, 128, 128, bits, 32)
+        gen = torch.Generator(device=cuda_device).manual_seed(bits)
+        tokens = 258 * spec.block_tokens - 3
+        k = torch.randn(tokens, spec.kv_heads, 128, generator=gen, device=cuda_device).to(dtype)
+        v = torch.randn(tokens, spec.kv_heads, 128, generator=gen, device=cuda_device).to(dtype)
+        recs, crcs = R.encode_records(k, v, spec, 3)
+        at = 0
+        for n in (200, 58):
+            span = slice(at * spec.block_tokens, (at + n) * spec.block_tokens)
+            part, part_crcs = R.encode_records(k[span], v[span], spec, 3, first_block=at)
+            assert torch.equal(recs[at : at + n], part) and torch.equal(crcs[at : at + n], part_crcs)
+            at += n
