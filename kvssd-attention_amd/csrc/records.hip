@@ -211,16 +211,7 @@ __device__ __forceinline__ void quantize_group(const T* src, int group_size, int
   *scale = __builtin_bit_cast(uint16_t, static_cast<_Float16>(s32));
 }
 
-// The same arithmetic for a 32-value group held in registers: the group is
-// read once with wide loads (src 16-byte aligned) and its packed bytes go out
-// in one 4-byte aligned store of 4 (INT4) or 2 (INT2) words.
-constexpr int kRegGroup = 32;
-
-template <int BITS>
-struct GroupWords {
-  uint32_t w[kRegGroup * BITS / 32];  // packed codes, low bits first
-  uint16_t scale;                     // fp16 bits
-};
+constexpr int kRegGroup = 32;  // the fused encode's group size
 
 // A word of codes, low bits first: clamp(rint(x / s32), -mid, mid - 1) + mid
 // with x / s32 rounded as IEEE division does, |x| <= (mid - 1) s32 (1 + 2^-23) or
@@ -274,58 +265,78 @@ __device__ __forceinline__ uint32_t code_word(const float (&x)[32 / BITS], float
   return static_cast<uint32_t>(half[0]) | (static_cast<uint32_t>(half[1]) << 16);
 }
 
-// max(amax, 1e-8) / (mid - 1), IEEE
+// max(amax, 1e-8) / (mid - 1), IEEE: a quotient by 7 lies at least 1/14 ulp from
+// the middle of two floats, which two roundings around 1/7 resolve (checked over
+// every mantissa); large values, where the remainder may not be finite, divide.
 template <int BITS>
 __device__ __forceinline__ float group_scale(float amax) {
-  return fmaxf(amax, 1e-8f) / static_cast<float>((1 << (BITS - 1)) - 1);
+  const float a = fmaxf(amax, 1e-8f);
+  if constexpr (BITS == 2) return a;
+  if (!(a < 0x1p120f)) return a / 7.0f;
+  const float q = a * (1.0f / 7.0f);
+  return __builtin_fmaf(__builtin_fmaf(-7.0f, q, a), 1.0f / 7.0f, q);
 }
 
+template <int CTRL>
+__device__ __forceinline__ float max_across(float v) {
+  return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true)));
+}
+
+// largest of v over each run of `lanes` (a power of two) lanes
+__device__ __forceinline__ float lanes_max(float v, int lanes) {
+  if (lanes > 1) v = max_across<0xB1>(v);    // lane ^ 1
+  if (lanes > 2) v = max_across<0x4E>(v);    // lane ^ 2
+  if (lanes > 4) v = max_across<0x141>(v);   // the other quad of 8
+  if (lanes > 8) v = max_across<0x140>(v);   // the other half of 16
+  for (int m = 16; m < lanes; m <<= 1) v = fmaxf(v, __shfl_xor(v, m, 64));
+  return v;
+}
+
+// The word form: a lane takes the 8 (INT4) or 16 (INT2) values of one word of
+// codes, `lanes` of them (a power of two) a group, so that loads and stores are
+// contiguous over the wave.  Measured (131,072 x 8 x
+// 128 bfloat16 keys and values into records, INT4): groups of 64, which went
+// through a thread a group with a load per value, 10.2 -> 0.23 ms; groups of 32
+// in 32-token blocks, before by a lane a group in registers, 0.31 -> 0.26 ms.
 template <typename T, int BITS>
-__device__ __forceinline__ GroupWords<BITS> quantize_group_words(const T* src) {
-  float x[kRegGroup];
-  if (src) {
-    T v[kRegGroup];
+__device__ __forceinline__ void quantize_word(const T* src, int lanes, uint8_t* packed, uint16_t* scale) {
+  constexpr int kVals = 32 / BITS;
+  float x[kVals], amax = 0.0f;
+  if (src != nullptr) {
+    T v[kVals];
     __builtin_memcpy(v, __builtin_assume_aligned(src, 16), sizeof(v));
 #pragma unroll
-    for (int i = 0; i < kRegGroup; ++i) x[i] = to_f32(v[i]);
+    for (int i = 0; i < kVals; ++i) x[i] = to_f32(v[i]);
   } else {
 #pragma unroll
-    for (int i = 0; i < kRegGroup; ++i) x[i] = 0.0f;
+    for (int i = 0; i < kVals; ++i) x[i] = 0.0f;
   }
-  float amax = 0.0f;
 #pragma unroll
-  for (int i = 0; i < kRegGroup; ++i) amax = fmaxf(amax, fabsf(x[i]));
-  const float s32 = group_scale<BITS>(amax);
-  GroupWords<BITS> g;
-#pragma unroll
-  for (int k = 0; k < BITS; ++k) {
-    float part[32 / BITS];
-#pragma unroll
-    for (int i = 0; i < 32 / BITS; ++i) part[i] = x[k * (32 / BITS) + i];
-    g.w[k] = code_word<T, BITS>(part, s32);
-  }
-  g.scale = __builtin_bit_cast(uint16_t, static_cast<_Float16>(s32));
-  return g;
+  for (int i = 0; i < kVals; ++i) amax = fmaxf(amax, fabsf(x[i]));
+  const float s32 = group_scale<BITS>(lanes_max(amax, lanes));
+  const uint32_t word = code_word<T, BITS>(x, s32);
+  __builtin_memcpy(__builtin_assume_aligned(packed, 4), &word, 4);
+  if ((threadIdx.x & (lanes - 1)) == 0) *scale = __builtin_bit_cast(uint16_t, static_cast<_Float16>(s32));
 }
 
-template <typename T, int BITS>
-__device__ __forceinline__ void quantize_group_reg(const T* src, uint8_t* packed, uint16_t* scale) {
-  const GroupWords<BITS> g = quantize_group_words<T, BITS>(src);
-  __builtin_memcpy(__builtin_assume_aligned(packed, 4), g.w, sizeof(g.w));
-  *scale = g.scale;
+// lanes of a group in the word form, 0 where it does not apply: whole words, a
+// power of two of them within a wave
+inline int word_lanes(int group_size, int bits) {
+  const int lanes = group_size * bits % 32 == 0 ? group_size * bits / 32 : 0;
+  return lanes <= 64 && (lanes & (lanes - 1)) == 0 ? lanes : 0;
 }
 
-// BITS == 0: any group size (quantize_group); BITS == 2 / 4: group_size 32
-// in registers (quantize_group_reg)
+// lanes == 0: a thread a group, any size and alignment (quantize_group);
+// else the word form, a thread a word
 template <typename T, int BITS>
-__global__ __launch_bounds__(256) void quantize_kernel(const T* __restrict__ x, int64_t groups, int group_size, int bits,
+__global__ __launch_bounds__(256) void quantize_kernel(const T* __restrict__ x, int64_t count, int group_size, int lanes,
                                                        uint8_t* __restrict__ packed, uint16_t* __restrict__ scales) {
-  const int64_t g = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (g >= groups) return;
-  if constexpr (BITS == 0) {
-    quantize_group(x + g * group_size, group_size, bits, packed + g * (group_size * bits / 8), scales + g);
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= count) return;
+  if (lanes == 0) {
+    quantize_group(x + i * group_size, group_size, BITS, packed + i * (group_size * BITS / 8), scales + i);
   } else {
-    quantize_group_reg<T, BITS>(x + g * kRegGroup, packed + g * (kRegGroup * BITS / 8), scales + g);
+    quantize_word<T, BITS>(x + i * (32 / BITS), lanes, packed + 4 * i, scales + i / lanes);
   }
 }
 
@@ -342,9 +353,8 @@ struct EncodeParams {
 };
 
 // phase 1: every (record, key/value, token, kv head, group) quantised into
-// the record's payload; tokens past the end read as zeros.  BITS as in
-// quantize_kernel.
-template <typename T, int BITS>
+// the record's payload; tokens past the end read as zeros.
+template <typename T>
 __global__ __launch_bounds__(256) void encode_payload_kernel(EncodeParams p) {
   const Layout& L = p.lay;
   const int G = L.head_dim / L.group_size;
@@ -365,11 +375,25 @@ __global__ __launch_bounds__(256) void encode_payload_kernel(EncodeParams p) {
   const int64_t s = L.scale_bytes(), pb = L.packed_bytes();
   uint16_t* scale = reinterpret_cast<uint16_t*>(pay + (is_v ? s : 0)) + q;
   uint8_t* packed = pay + 2 * s + (is_v ? pb : 0) + q * (L.group_size * L.bits / 8);
-  if constexpr (BITS == 0) {
-    quantize_group(src, L.group_size, L.bits, packed, scale);
-  } else {
-    quantize_group_reg<T, BITS>(src, packed, scale);
-  }
+  quantize_group(src, L.group_size, L.bits, packed, scale);
+}
+
+// phase 1 in the word form: grid y is (record, key/value), whose values and
+// words lie in one run each
+template <typename T, int BITS>
+__global__ __launch_bounds__(256) void encode_words_kernel(EncodeParams p, int lanes) {
+  const Layout& L = p.lay;
+  const int64_t w = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;  // of the array
+  const int64_t s = L.scale_bytes(), pb = L.packed_bytes();
+  if (4 * w >= pb) return;
+  const int r = static_cast<int>(blockIdx.y >> 1);
+  const bool is_v = blockIdx.y & 1;
+  const int64_t row = static_cast<int64_t>(L.kv_heads) * L.head_dim;
+  const int64_t at = r * (L.block_tokens * row) + w * (32 / BITS);  // of the layer's values
+  const T* base = static_cast<const T*>(is_v ? p.values : p.keys);
+  uint8_t* pay = p.records + static_cast<int64_t>(r) * L.record_bytes() + kHeaderBytes;
+  quantize_word<T, BITS>(at < p.tokens * row ? base + at : nullptr, lanes, pay + 2 * s + (is_v ? pb : 0) + 4 * w,
+                         reinterpret_cast<uint16_t*>(pay + (is_v ? s : 0)) + w / lanes);
 }
 
 // phase 2: one workgroup per record -- CRC of the payload, header, padding.
@@ -459,15 +483,6 @@ struct FusedPlan {
 constexpr int kComputeUnits = 256;
 constexpr int kMaxScaleRows = kGroupRows;  // scale region <= 64 KiB of LDS, one group of rows
 
-// largest of v over the BITS lanes (4 or 2) that share a group
-template <int BITS>
-__device__ __forceinline__ float group_max(float v) {
-  v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true)));
-  if constexpr (BITS == 4)
-    v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, true)));
-  return v;
-}
-
 // PARTS: the workgroup has 1024 / PARTS threads, each taking the parts of PARTS
 // in turn.
 template <typename T, int BITS, int PARTS>
@@ -544,7 +559,7 @@ __global__ __launch_bounds__(kCrcThreads / PARTS) void encode_fused_kernel(Encod
               x[i] = to_f32(v[i]);
               amax = fmaxf(amax, fabsf(x[i]));
             }
-            const float s32 = group_scale<BITS>(group_max<BITS>(amax));
+            const float s32 = group_scale<BITS>(lanes_max(amax, BITS));
             const uint32_t word = code_word<T, BITS>(x, s32);
             words[u] = word;
             if ((lane & (BITS - 1)) == 0)
@@ -610,7 +625,7 @@ __global__ __launch_bounds__(kCrcThreads / PARTS) void encode_fused_kernel(Encod
   if (tid == 0) p.crcs[r] = crc;
 }
 
-// the fused form applies (register groups checked separately): scale and code
+// the fused form applies: scale and code
 // regions whole rows of the chunked CRC form, scales within the LDS copy
 bool fused_layout(const Layout& L, FusedPlan* f) {
   const int64_t sr = 2 * L.scale_bytes(), cr = 2 * L.packed_bytes();
@@ -638,25 +653,22 @@ int check_layout(const kvssd_record_layout* l, Layout* out) {
   return 0;
 }
 
-// the register form needs group_size 32, a 16-byte aligned source and 4-byte
-// aligned packed output (every group then starts aligned)
-inline bool register_groups(int group_size, const void* src, const void* packed) {
-  return group_size == kRegGroup && (reinterpret_cast<uintptr_t>(src) & 15u) == 0 &&
-         (reinterpret_cast<uintptr_t>(packed) & 3u) == 0;
+// the word form's loads and stores: a 16-byte aligned source, 4-byte aligned codes
+inline bool word_aligned(const void* src, const void* packed) {
+  return (reinterpret_cast<uintptr_t>(src) & 15u) == 0 && (reinterpret_cast<uintptr_t>(packed) & 3u) == 0;
 }
 
 template <typename T>
 void launch_quantize_t(const void* x, int64_t groups, int group_size, int bits, uint8_t* packed, uint16_t* scales,
                        hipStream_t s) {
-  const dim3 grid(static_cast<unsigned>((groups + 255) / 256));
+  const int lanes = word_aligned(x, packed) ? word_lanes(group_size, bits) : 0;
+  const int64_t count = lanes > 0 ? groups * lanes : groups;
+  const dim3 grid(static_cast<unsigned>((count + 255) / 256));
   const T* src = static_cast<const T*>(x);
-  if (register_groups(group_size, x, packed) && bits == 4) {
-    hipLaunchKernelGGL((quantize_kernel<T, 4>), grid, dim3(256), 0, s, src, groups, group_size, bits, packed, scales);
-  } else if (register_groups(group_size, x, packed) && bits == 2) {
-    hipLaunchKernelGGL((quantize_kernel<T, 2>), grid, dim3(256), 0, s, src, groups, group_size, bits, packed, scales);
-  } else {
-    hipLaunchKernelGGL((quantize_kernel<T, 0>), grid, dim3(256), 0, s, src, groups, group_size, bits, packed, scales);
-  }
+  if (bits == 4)
+    hipLaunchKernelGGL((quantize_kernel<T, 4>), grid, dim3(256), 0, s, src, count, group_size, lanes, packed, scales);
+  else
+    hipLaunchKernelGGL((quantize_kernel<T, 2>), grid, dim3(256), 0, s, src, count, group_size, lanes, packed, scales);
 }
 
 template <typename T, int PARTS>
@@ -684,15 +696,16 @@ template <typename T>
 void launch_encode_t(const EncodeParams& p, hipStream_t s) {
   const int64_t groups = 2LL * p.lay.block_tokens * p.lay.kv_heads * (p.lay.head_dim / p.lay.group_size) * p.n;
   const dim3 grid(static_cast<unsigned>((groups + 255) / 256));
-  // records are 4-byte aligned (checked), so every packed group is too
-  const bool reg = register_groups(p.lay.group_size, p.keys, p.records) &&
-                   (reinterpret_cast<uintptr_t>(p.values) & 15u) == 0;
-  if (reg && p.lay.bits == 4) {
-    hipLaunchKernelGGL((encode_payload_kernel<T, 4>), grid, dim3(256), 0, s, p);
-  } else if (reg && p.lay.bits == 2) {
-    hipLaunchKernelGGL((encode_payload_kernel<T, 2>), grid, dim3(256), 0, s, p);
+  const int lanes = word_lanes(p.lay.group_size, p.lay.bits);
+  // (records are 4-byte aligned, checked; the codes after them too where the scales are whole words; grid y holds 65,535)
+  if (lanes > 0 && word_aligned(p.keys, p.records) && word_aligned(p.values, p.records) &&
+      2 * p.lay.scale_bytes() % 4 == 0 && p.lay.packed_bytes() % 4 == 0 && p.n <= 32767 &&
+      p.lay.block_tokens * p.lay.kv_heads * static_cast<int64_t>(p.lay.head_dim) % 16 == 0) {
+    const dim3 words(static_cast<unsigned>((p.lay.packed_bytes() / 4 + 255) / 256), static_cast<unsigned>(2 * p.n));
+    if (p.lay.bits == 4) hipLaunchKernelGGL((encode_words_kernel<T, 4>), words, dim3(256), 0, s, p, lanes);
+    else hipLaunchKernelGGL((encode_words_kernel<T, 2>), words, dim3(256), 0, s, p, lanes);
   } else {
-    hipLaunchKernelGGL((encode_payload_kernel<T, 0>), grid, dim3(256), 0, s, p);
+    hipLaunchKernelGGL(encode_payload_kernel<T>, grid, dim3(256), 0, s, p);
   }
 }
 
@@ -796,8 +809,7 @@ int launch_encode_records(const kvssd_record_layout* layout, int dtype, const vo
   const ChunkPlan c = make_chunk_plan(len);
   FusedPlan f{};
   // (fp64 input keeps the two-kernel form: its fused INT2 instance would spill)
-  if (fused_layout(L, &f) && register_groups(L.group_size, keys, records) &&
-      (reinterpret_cast<uintptr_t>(values) & 15u) == 0 &&
+  if (fused_layout(L, &f) && word_aligned(keys, records) && word_aligned(values, records) &&
       (dtype == KVSSD_DTYPE_F16 || dtype == KVSSD_DTYPE_BF16 || dtype == KVSSD_DTYPE_F32)) {
     if (dtype == KVSSD_DTYPE_F16) launch_fused_t<_Float16>(p, c, f, stream);
     else if (dtype == KVSSD_DTYPE_BF16) launch_fused_t<uint16_t>(p, c, f, stream);

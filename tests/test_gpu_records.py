@@ -323,3 +323,24 @@ def test_encode_more_records_than_compute_units(cuda_device, bits, dtype):
             part, part_crcs = R.encode_records(k[span], v[span], spec, 3, first_block=at)
             assert torch.equal(recs[at : at + n], part) and torch.equal(crcs[at : at + n], part_crcs)
             at += n
+
+
+@pytest.mark.parametrize("bits", [2, 4])
+@pytest.mark.parametrize("g", [8, 16, 24, 64, 128, 256])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float64])
+def test_word_form_group_sizes(cuda_device, bits, g, dtype):
+    # groups of one to 32 lanes of a word each, and sizes that are not (INT2 of 8, 24): rows
+    # that end inside a workgroup, a last record partly filled; the oracle's bytes
+    d = 2 * g if g >= 64 else 6 * g
+    gen = torch.Generator().manual_seed(g)
+    x = torch.randn(37, d, generator=gen).to(dtype)
+    q = R.quantize(x.to(cuda_device), bits, g)
+    packed, scales = oracle_quantize(x, bits, g)
+    assert np.array_equal(q.packed.cpu().numpy(), packed)
+    assert np.array_equal(q.scales.cpu().numpy().view(np.uint16), scales.view(np.uint16))
+    spec = CacheSpec(1, 3, d, 21, bits, g)
+    k = torch.randn(50, 3, d, generator=gen).to(dtype)
+    v = torch.randn(50, 3, d, generator=gen).to(dtype)
+    recs, _ = R.encode_records(k.to(cuda_device), v.to(cuda_device), spec, 2, 4)
+    want = oracle_records(k.float().numpy(), v.float().numpy(), spec, 2, 4)
+    assert [r.tobytes() for r in recs.cpu().numpy()] == want
