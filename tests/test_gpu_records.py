@@ -344,3 +344,35 @@ def test_word_form_group_sizes(cuda_device, bits, g, dtype):
     recs, _ = R.encode_records(k.to(cuda_device), v.to(cuda_device), spec, 2, 4)
     want = oracle_records(k.float().numpy(), v.float().numpy(), spec, 2, 4)
     assert [r.tobytes() for r in recs.cpu().numpy()] == want
+
+
+def test_encode_more_records_than_a_grid(cuda_device):
+    # past 32,767 records the two-pass encode takes several launches: the same bytes and CRC
+    # values as two calls of half the records, the last one partly filled, and no slower
+    # kernel for them (one record more than a launch holds took ten times as long)
+    spec = CacheSpec(1, 4, 64, 16, 4, 32)
+    n = 32769
+    gen = torch.Generator(device=cuda_device).manual_seed(1)
+    k = torch.randn(n * 16 - 5, 4, 64, generator=gen, device=cuda_device).half()
+    v = torch.randn(n * 16 - 5, 4, 64, generator=gen, device=cuda_device).half()
+    recs, crcs = R.encode_records(k, v, spec, 3)
+    at = 0
+    for m in (16384, 16385):
+        span = slice(at * 16, (at + m) * 16)
+        part, part_crcs = R.encode_records(k[span], v[span], spec, 3, first_block=at)
+        assert torch.equal(recs[at : at + m], part) and torch.equal(crcs[at : at + m], part_crcs)
+        at += m
+    del recs, crcs, part
+
+    def fastest(tokens):
+        times = []
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            R.encode_records(k[:tokens], v[:tokens], spec, 3)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    assert fastest(n * 16 - 5) < 1.5 * fastest(32767 * 16)
