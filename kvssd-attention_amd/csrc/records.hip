@@ -481,6 +481,7 @@ struct FusedPlan {
 };
 
 constexpr int kComputeUnits = 256;
+constexpr int kLdsBytes = 160 * 1024;  // of a CU
 constexpr int kMaxScaleRows = kGroupRows;  // scale region <= 64 KiB of LDS, one group of rows
 
 // PARTS: the workgroup has 1024 / PARTS threads, each taking the parts of PARTS
@@ -685,11 +686,26 @@ void launch_fused_parts(const EncodeParams& p, const ChunkPlan& c, const FusedPl
 // share a CU, and one's start and end pass under the other's work (128-token
 // records of 8 kv heads: 257 of them 71 -> 66 us a call, 400 79 -> 74, 1,024
 // 174 -> 170).  Up to there 1024 threads finish a record sooner (256: 42 us
-// against 47, 16: 33 against 37).
+// against 47, 16: 33 against 37), and so they do where the LDS of two does not
+// fit a CU (64 KiB of scales, 32 kv heads: 300 records 256 us against 338, 600
+// 404 against 518).
 template <typename T>
 void launch_fused_t(const EncodeParams& p, const ChunkPlan& c, const FusedPlan& f, hipStream_t s) {
-  if (p.n > kComputeUnits) launch_fused_parts<T, 2>(p, c, f, s);
+  const bool two_fit = 2 * (2 * p.lay.scale_bytes() + static_cast<int64_t>(sizeof(ChunkLds))) <= kLdsBytes;
+  if (p.n > kComputeUnits && two_fit) launch_fused_parts<T, 2>(p, c, f, s);
   else launch_fused_parts<T, 1>(p, c, f, s);
+}
+
+// One workgroup a record pays off while a record is short, or where records
+// fill the chip.  Past 8 code rows (8 kv heads of 128 tokens, INT4) the two
+// passes, which spread a record over the chip, are faster for few records (16
+// kv heads, INT4, bfloat16: 64 records 39 us against 58, 256 103 against 82;
+// 32 heads: 64 64 against 102, 600 461 against 404), and at any count for INT2
+// codes or fp32 values, whose quantising outweighs the payload read back (24
+// kv heads, 300 records: INT2 bfloat16 124 us against 158, fp32 211 against
+// 288; INT4 fp32 238 against 294).
+bool fused_pays(const FusedPlan& f, int bits, int dtype, int n) {
+  return f.rows_c <= 8 || (bits == 4 && dtype != KVSSD_DTYPE_F32 && n > kComputeUnits / 2);
 }
 
 // records of one launch of the word form, whose (record, key/value) pairs are
@@ -824,7 +840,7 @@ int launch_encode_records(const kvssd_record_layout* layout, int dtype, const vo
   const ChunkPlan c = make_chunk_plan(len);
   FusedPlan f{};
   // (fp64 input keeps the two-kernel form: its fused INT2 instance would spill)
-  if (fused_layout(L, &f) && word_aligned(keys, records) && word_aligned(values, records) &&
+  if (fused_layout(L, &f) && fused_pays(f, L.bits, dtype, p.n) && word_aligned(keys, records) && word_aligned(values, records) &&
       (dtype == KVSSD_DTYPE_F16 || dtype == KVSSD_DTYPE_BF16 || dtype == KVSSD_DTYPE_F32)) {
     if (dtype == KVSSD_DTYPE_F16) launch_fused_t<_Float16>(p, c, f, stream);
     else if (dtype == KVSSD_DTYPE_BF16) launch_fused_t<uint16_t>(p, c, f, stream);

@@ -376,3 +376,47 @@ def test_encode_more_records_than_a_grid(cuda_device):
         return min(times)
 
     assert fastest(n * 16 - 5) < 1.5 * fastest(32767 * 16)
+
+
+@pytest.mark.parametrize(("kvh", "bits", "dtype"), [(24, 4, torch.bfloat16), (32, 4, torch.float16), (32, 4, torch.float32),
+                                                    (24, 2, torch.float32), (32, 2, torch.bfloat16)])
+def test_encode_wide_layers(cuda_device, kvh, bits, dtype):
+    # three and four rows of scales, up to the most LDS a workgroup takes: few records (two passes),
+    # more than half a CU's worth each and more than one (16-bit INT4: one kernel); the oracle's
+    # bytes for few, and the same bytes in larger calls
+    spec = CacheSpec(1, kvh, 128, 128, bits, 32)
+    gen = torch.Generator(device=cuda_device).manual_seed(kvh + bits)
+    tokens = 258 * 128 - 3
+    k = torch.randn(tokens, kvh, 128, generator=gen, device=cuda_device).to(dtype)
+    v = torch.randn(tokens, kvh, 128, generator=gen, device=cuda_device).to(dtype)
+    parts = [R.encode_records(k[a * 128 : b * 128], v[a * 128 : b * 128], spec, 1, a) for a, b in ((0, 128), (128, 255), (255, 258))]
+    want = oracle_records(k[255 * 128 :].float().cpu().numpy(), v[255 * 128 :].float().cpu().numpy(), spec, 1, 255)
+    assert [r.tobytes() for r in parts[2][0].cpu().numpy()] == want
+    recs, crcs = (torch.cat([p[i] for p in parts]) for i in (0, 1))
+    for n in (129, 256, 258):
+        got, got_crcs = R.encode_records(k[: n * 128], v[: n * 128], spec, 1)
+        assert torch.equal(got, recs[:n]) if n == 258 else torch.equal(got[: n - 1], recs[: n - 1])
+        assert torch.equal(got_crcs[: n - 1], crcs[: n - 1])
+        host = got[n - 1].cpu().numpy()
+        assert int(got_crcs[n - 1]) == zlib.crc32(host[52 : 52 + int.from_bytes(host[44:48].tobytes(), "little")].tobytes())
+
+
+def test_encode_wide_layers_few_records_keep_their_speed(cuda_device):
+    # a layer of 24 kv heads, INT2 of fp32 values, 64 records: one workgroup a record takes about
+    # twice the time that the same values take as 24 records' worth of smaller blocks in two passes
+    def fastest(spec, dtype):
+        k = torch.randn(64 * 128, 24, 128, device=cuda_device).to(dtype)
+        times = []
+        R.encode_records(k, k, spec, 0)
+        for _ in range(8):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(4):
+                R.encode_records(k, k, spec, 0)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    small = fastest(CacheSpec(1, 24, 128, 64, 2, 32), torch.float32)
+    assert fastest(CacheSpec(1, 24, 128, 128, 2, 32), torch.float32) < 1.4 * small
