@@ -104,6 +104,13 @@ int kvssd_hip_decode_workspace_bytes(const kvssd_decode_desc* desc, size_t* byte
  * never KVSSD_KERNEL_AUTO). */
 int kvssd_hip_decode_kernel(const kvssd_decode_desc* desc, int* kernel);
 
+/* What kvssd_hip_fused_decode launches for `desc` and arrays at these addresses
+ * (of which only the alignment counts; nothing is read): the kernel, *tiled = 1
+ * where KVSSD_KERNEL_GENERAL is answered by the tiled matrix-core kernel and
+ * not by the vector one, and the number of splits whose partials it merges. */
+int kvssd_hip_decode_plan(const kvssd_decode_desc* desc, const uint8_t* packed_k, const uint8_t* packed_v,
+                          const uint16_t* scales_k, const uint16_t* scales_v, int* kernel, int* tiled, int* splits);
+
 /* Fused decode attention over a packed batch: out [query_heads, head_dim]
  * (softmax-normalised; fp32, or query_dtype with desc->out_query_dtype = 1),
  * lse fp32 [query_heads] (natural-log log-sum-exp of the

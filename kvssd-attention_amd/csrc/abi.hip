@@ -120,10 +120,10 @@ int units_of_desc(const kvssd_decode_desc* d, int* units) {
 int plan_checked(const kvssd_decode_desc* desc, int units, const void* workspace, size_t workspace_bytes, int* kernel,
                  int* splits) {
   if (int rc = choose_kernel(*desc, kernel)) return rc;
-  const size_t need = split_partial_bytes(plan_splits(*desc, units).splits, desc->query_heads, desc->head_dim);
+  *splits = plan_splits(*desc, units).splits;
+  const size_t need = split_partial_bytes(*splits, desc->query_heads, desc->head_dim);
   if (workspace == nullptr || workspace_bytes < need)
     return arg_error("workspace too small: need " + std::to_string(need) + " bytes");
-  *splits = launch_splits(*desc, units).splits;
   return 0;
 }
 
@@ -168,6 +168,37 @@ int static_scratch(void** ptr) {
 // Element type of `out`: fp32, or the query's dtype when the caller asks.
 int out_dtype_of(const kvssd_decode_desc& d) { return d.out_query_dtype ? d.query_dtype : KVSSD_DTYPE_F32; }
 
+// The kernel that runs on arrays at these addresses, and its splits.  Where the
+// tiled kernel runs it takes fewer than the plan_splits that the workspace is
+// sized for.  (The shapes that the matrix-core kernels take keep plan_splits.)
+bool fewer_splits(const kvssd_decode_desc& d) { return tile_supported(d) && !mfma_supported(d, nullptr); }
+
+struct Launch {
+  int kernel;
+  bool tiled;  // KVSSD_KERNEL_GENERAL answered by the tiled matrix-core kernel
+  SplitPlan plan;
+};
+
+int resolve_launch(const DecodeArgs& a, int kernel, Launch* out) {
+  const kvssd_decode_desc& d = a.desc;
+  if (kernel == KVSSD_KERNEL_STAGED && !staged_aligned(a)) {
+    if (d.kernel == KVSSD_KERNEL_STAGED)
+      return arg_error("staged matrix-core kernel needs 16-byte aligned packed arrays and scales");
+    kernel = KVSSD_KERNEL_MFMA;
+  }
+  if (kernel == KVSSD_KERNEL_MFMA && !mfma_aligned(a)) {
+    if (d.kernel == KVSSD_KERNEL_MFMA)
+      return arg_error(
+          "matrix-core kernel needs 16-byte aligned packed arrays (8-byte for INT2) and 8-byte aligned scales");
+    kernel = KVSSD_KERNEL_GENERAL;
+  }
+  out->kernel = kernel;
+  out->tiled = kernel == KVSSD_KERNEL_GENERAL && tile_supported(d) && tile_aligned(a);
+  out->plan = plan_splits(d, a.units);
+  if (out->tiled && fewer_splits(d)) out->plan = tile_splits(d, a.units, out->plan);
+  return 0;
+}
+
 // Both decode entry points: the split kernel, then (with `out`) the merge.
 int decode_call(const kvssd_decode_desc* desc, const void* query, const uint8_t* packed_k, const uint8_t* packed_v,
                 const uint16_t* scales_k, const uint16_t* scales_v, const int32_t* valid_tokens,
@@ -188,25 +219,20 @@ int decode_call(const kvssd_decode_desc* desc, const void* query, const uint8_t*
   a.table = block_table;
   a.units = units;
   a.stream = static_cast<hipStream_t>(stream);
-  SplitPartials parts = carve_partials(workspace, splits, desc->query_heads, desc->head_dim);
-  const SplitPlan plan = launch_splits(*desc, units);
-  if (kernel == KVSSD_KERNEL_STAGED && !staged_aligned(a)) {
-    if (desc->kernel == KVSSD_KERNEL_STAGED)
-      return arg_error("staged matrix-core kernel needs 16-byte aligned packed arrays and scales");
-    kernel = KVSSD_KERNEL_MFMA;
-  }
-  if (kernel == KVSSD_KERNEL_MFMA && !mfma_aligned(a)) {
-    if (desc->kernel == KVSSD_KERNEL_MFMA)
-      return arg_error(
-          "matrix-core kernel needs 16-byte aligned packed arrays (8-byte for INT2) and 8-byte aligned scales");
-    kernel = KVSSD_KERNEL_GENERAL;
-  }
-  int rc = kernel == KVSSD_KERNEL_STAGED ? launch_staged(a, plan, parts)
-           : kernel == KVSSD_KERNEL_MFMA ? launch_mfma(a, plan, parts)
-                                         : launch_general(a, plan, parts);
-  if (rc != 0 || out == nullptr) return rc;
-  return launch_merge_splits(parts, splits, desc->query_heads, desc->head_dim, out, out_dtype_of(*desc), lse,
-                             a.stream);
+  Launch l{};
+  if (int rc = resolve_launch(a, kernel, &l)) return rc;
+  // a merge in a call of its own knows plan_splits only: the partials are laid
+  // out for those, and the tiled kernel leaves word of its fewer splits
+  const bool separate = out == nullptr;
+  SplitPartials parts = carve_partials(workspace, separate ? splits : l.plan.splits, desc->query_heads, desc->head_dim);
+  if (separate && l.plan.splits < splits) a.split_note = split_note(parts, splits, desc->query_heads);
+  int rc = l.kernel == KVSSD_KERNEL_STAGED ? launch_staged(a, l.plan, parts)
+           : l.kernel == KVSSD_KERNEL_MFMA ? launch_mfma(a, l.plan, parts)
+           : l.tiled                       ? launch_tile(a, l.plan, parts)
+                                           : launch_general(a, l.plan, parts);
+  if (rc != 0 || separate) return rc;
+  return launch_merge_splits(parts, l.plan.splits, false, desc->query_heads, desc->head_dim, out, out_dtype_of(*desc),
+                             lse, a.stream);
 }
 
 }  // namespace
@@ -272,6 +298,30 @@ __attribute__((visibility("default"))) int kvssd_hip_decode_kernel(const kvssd_d
   return choose_kernel(*desc, kernel);
 }
 
+__attribute__((visibility("default"))) int kvssd_hip_decode_plan(const kvssd_decode_desc* desc,
+                                                                 const uint8_t* packed_k, const uint8_t* packed_v,
+                                                                 const uint16_t* scales_k, const uint16_t* scales_v,
+                                                                 int* kernel, int* tiled, int* splits) {
+  int units = 0, chosen = 0;
+  if (int rc = validate(desc, &units)) return rc;
+  if (kernel == nullptr || tiled == nullptr || splits == nullptr) return arg_error("an output pointer is NULL");
+  if (int rc = units_of_desc(desc, &units)) return rc;
+  if (int rc = choose_kernel(*desc, &chosen)) return rc;
+  DecodeArgs a{};
+  a.desc = *desc;
+  a.packed_k = packed_k;
+  a.packed_v = packed_v;
+  a.scales_k = scales_k;
+  a.scales_v = scales_v;
+  a.units = units;
+  Launch l{};
+  if (int rc = resolve_launch(a, chosen, &l)) return rc;
+  *kernel = l.kernel;
+  *tiled = l.tiled ? 1 : 0;
+  *splits = l.plan.splits;
+  return 0;
+}
+
 __attribute__((visibility("default"))) int kvssd_hip_decode_workspace_bytes(const kvssd_decode_desc* desc,
                                                                             size_t* bytes) {
   int units = 0;
@@ -301,8 +351,8 @@ __attribute__((visibility("default"))) int kvssd_hip_decode_merge(const kvssd_de
   if (int rc = plan_checked(desc, units, workspace, workspace_bytes, &kernel, &splits)) return rc;
   if (!out || !lse) return arg_error("a required buffer pointer is NULL");
   SplitPartials parts = carve_partials(const_cast<void*>(workspace), splits, desc->query_heads, desc->head_dim);
-  return launch_merge_splits(parts, splits, desc->query_heads, desc->head_dim, out, out_dtype_of(*desc), lse,
-                             static_cast<hipStream_t>(stream));
+  return launch_merge_splits(parts, splits, fewer_splits(*desc), desc->query_heads, desc->head_dim, out,
+                             out_dtype_of(*desc), lse, static_cast<hipStream_t>(stream));
 }
 
 __attribute__((visibility("default"))) int kvssd_hip_fused_decode(

@@ -16,6 +16,7 @@ struct DecodeArgs {
   const int32_t* table;  // nullptr: identity over num_blocks
   int units;             // blocks attended (num_selected or num_blocks)
   hipStream_t stream;
+  float* split_note;     // where the tiled kernel notes its splits (split_note), or nullptr
 };
 
 // ---- kernel arguments of the matrix-core kernels.  Their first nine
@@ -52,18 +53,19 @@ struct SplitPlan {
   int splits;            // partitions of the attended blocks
   int blocks_per_split;  // consecutive attended blocks per partition
 };
-// the most splits a shape's partials take (the workspace size)
+// (the tiled kernel takes fewer: tile_splits)
 SplitPlan plan_splits(const kvssd_decode_desc& d, int units);
-// the splits its launches and its merge use: those, or the tiled kernel's
-// fewer ones for the shapes only it and the general kernel take
-SplitPlan launch_splits(const kvssd_decode_desc& d, int units);
 
 // ---- general kernel: any head_dim <= 256, group size, GQA ratio, block size
 int launch_general(const DecodeArgs& a, const SplitPlan& plan, SplitPartials parts);
 
 // ---- tiled matrix-core kernel: the general kernel's fp32-grade arithmetic for head_dim 64 / 96 (INT4) / 128 / 256
 bool tile_supported(const kvssd_decode_desc& d);
+inline float* split_note(SplitPartials parts, int splits, int query_heads) {
+  return parts.ml + 2 * (static_cast<size_t>(splits - 1) * query_heads) + 1;  // an l, which is never negative
+}
 bool tile_aligned(const DecodeArgs& a);
+// its splits: at most `most`, which the workspace holds
 SplitPlan tile_splits(const kvssd_decode_desc& d, int units, const SplitPlan& most);
 int launch_tile(const DecodeArgs& a, const SplitPlan& plan, SplitPartials parts);
 
@@ -81,8 +83,10 @@ bool staged_aligned(const DecodeArgs& a);
 int launch_staged(const DecodeArgs& a, const SplitPlan& plan, SplitPartials parts);
 
 // ---- split-K phase 2: merge the partials of every split into (out, lse);
-// out holds elements of out_dtype (enum kvssd_dtype), lse fp32
-int launch_merge_splits(SplitPartials parts, int splits, int query_heads, int head_dim, void* out, int out_dtype,
+// out holds elements of out_dtype (enum kvssd_dtype), lse fp32.
+// noted: the partials are laid out for `splits` of which the decode may have
+// filled fewer; then the last one's l of head 0 holds minus their number.
+int launch_merge_splits(SplitPartials parts, int splits, bool noted, int query_heads, int head_dim, void* out, int out_dtype,
                         float* lse, hipStream_t stream);
 
 // ---- chunk merge (pipeline), codec twins

@@ -200,14 +200,8 @@ SplitPlan plan_splits(const kvssd_decode_desc& d, int units) {
   return plan;
 }
 
-SplitPlan launch_splits(const kvssd_decode_desc& d, int units) {
-  const SplitPlan most = plan_splits(d, units);
-  return tile_supported(d) && !mfma_supported(d, nullptr) ? tile_splits(d, units, most) : most;
-}
-
 int launch_general(const DecodeArgs& a, const SplitPlan& plan, SplitPartials parts) {
   const kvssd_decode_desc& d = a.desc;
-  if (tile_supported(d) && tile_aligned(a)) return launch_tile(a, plan, parts);
   const int gq = d.query_heads / d.kv_heads;
   const int heads_per_chunk = gq < kMaxHeads ? gq : kMaxHeads;
   const int head_chunks = (gq + heads_per_chunk - 1) / heads_per_chunk;

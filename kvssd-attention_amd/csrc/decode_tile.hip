@@ -54,6 +54,7 @@ struct TileTail {
   const int32_t* valid;
   float* part_o;
   float* part_ml;
+  float* split_note;                   // where to note `splits`, or nullptr
   int query_heads, num_blocks, gq, heads_per_wg;
   int head_chunks, query_dtype, splits;
   uint32_t chunk_magic;                // ceil(2^32 / head_chunks), head_chunks > 1
@@ -685,6 +686,7 @@ __global__ __launch_bounds__(kTileThreads, tile_workgroups_per_cu(D, HS, QSPLIT)
     r.part_ml[2 * (prow + tid)] = big;
     r.part_ml[2 * (prow + tid) + 1] = l;
   }
+  if (r.split_note != nullptr && split == 0 && blockIdx.y == 0 && tid == 0) *r.split_note = -static_cast<float>(r.splits);
 }
 
 int ceil_log2(int n) {
@@ -791,6 +793,7 @@ int launch_tile(const DecodeArgs& a, const SplitPlan& plan, SplitPartials parts)
   r.head_chunks = chunks;
   r.query_dtype = d.query_dtype;
   r.splits = plan.splits;
+  r.split_note = a.split_note;
   r.chunk_magic = chunks > 1 ? static_cast<uint32_t>(((1ull << 32) + chunks - 1) / chunks) : 0u;
   r.bt_magic = d.block_tokens < 256 ? ((1u << 20) + d.block_tokens - 1) / d.block_tokens : 0u;
   r.group_magic = (65536u + d.group_size - 1) / d.group_size;

@@ -44,7 +44,8 @@ constexpr int kMaxMergeSplits = 2048;
 constexpr int kSliceDims = 16;
 constexpr int kPhases = kWave / kSliceDims;  // 4
 
-template <int OPL, typename OFF, typename OT>
+// NOTED: the splits filled may be fewer than `splits` (see launch_merge_splits)
+template <int OPL, bool NOTED, typename OFF, typename OT>
 __global__ __launch_bounds__(kWave) void merge_splits_kernel(const float* __restrict__ part_o,
                                                             const float* __restrict__ part_ml, int splits,
                                                             int query_heads, int head_dim, OT* __restrict__ out,
@@ -53,6 +54,10 @@ __global__ __launch_bounds__(kWave) void merge_splits_kernel(const float* __rest
   constexpr int kOPerLane = OPL;
   constexpr int kMlPerLane = kBatchSplits / kWave;
   __shared__ float sw[kBatchSplits];  // [phase][j]: weight of split phase + 4 j of the batch
+  if constexpr (NOTED) {
+    const float note = part_ml[2 * (static_cast<size_t>(splits - 1) * query_heads) + 1];
+    if (note < 0.0f) splits = static_cast<int>(-note);
+  }
   const int h = blockIdx.x;
   const int d0 = blockIdx.y * kSliceDims;
   const int lane = threadIdx.x;
@@ -164,37 +169,44 @@ __global__ __launch_bounds__(kMergeThreads) void merge_chunks_kernel(int dim, fl
 
 }  // namespace
 
-template <typename OT>
+template <bool NOTED, typename OT>
 void launch_merge_typed(SplitPartials parts, int splits, int query_heads, int head_dim, OT* out, float* lse,
                         hipStream_t stream) {
   const int slices = (head_dim + kSliceDims - 1) / kSliceDims;
   const dim3 grid(query_heads, slices);
   if (split_partial_bytes(splits, query_heads, head_dim) > 0xFFFFFFFFull)
-    hipLaunchKernelGGL((merge_splits_kernel<16, uint64_t, OT>), grid, dim3(kWave), 0, stream, parts.o, parts.ml,
+    hipLaunchKernelGGL((merge_splits_kernel<16, NOTED, uint64_t, OT>), grid, dim3(kWave), 0, stream, parts.o, parts.ml,
                        splits, query_heads, head_dim, out, lse);
   else if (splits <= kPhases * 16)
-    hipLaunchKernelGGL((merge_splits_kernel<16, uint32_t, OT>), grid, dim3(kWave), 0, stream, parts.o, parts.ml,
+    hipLaunchKernelGGL((merge_splits_kernel<16, NOTED, uint32_t, OT>), grid, dim3(kWave), 0, stream, parts.o, parts.ml,
                        splits, query_heads, head_dim, out, lse);
   else
-    hipLaunchKernelGGL((merge_splits_kernel<64, uint32_t, OT>), grid, dim3(kWave), 0, stream, parts.o, parts.ml,
+    hipLaunchKernelGGL((merge_splits_kernel<64, NOTED, uint32_t, OT>), grid, dim3(kWave), 0, stream, parts.o, parts.ml,
                        splits, query_heads, head_dim, out, lse);
 }
 
-int launch_merge_splits(SplitPartials parts, int splits, int query_heads, int head_dim, void* out, int out_dtype,
+template <typename OT>
+void launch_merge_as(SplitPartials parts, int splits, bool noted, int query_heads, int head_dim, void* out, float* lse,
+                     hipStream_t stream) {
+  if (noted) launch_merge_typed<true>(parts, splits, query_heads, head_dim, static_cast<OT*>(out), lse, stream);
+  else launch_merge_typed<false>(parts, splits, query_heads, head_dim, static_cast<OT*>(out), lse, stream);
+}
+
+int launch_merge_splits(SplitPartials parts, int splits, bool noted, int query_heads, int head_dim, void* out, int out_dtype,
                         float* lse, hipStream_t stream) {
   if (splits > kMaxMergeSplits) return arg_error("too many splits for the merge kernel");
   switch (out_dtype) {
     case KVSSD_DTYPE_F16:
-      launch_merge_typed(parts, splits, query_heads, head_dim, static_cast<_Float16*>(out), lse, stream);
+      launch_merge_as<_Float16>(parts, splits, noted, query_heads, head_dim, out, lse, stream);
       break;
     case KVSSD_DTYPE_BF16:
-      launch_merge_typed(parts, splits, query_heads, head_dim, static_cast<uint16_t*>(out), lse, stream);
+      launch_merge_as<uint16_t>(parts, splits, noted, query_heads, head_dim, out, lse, stream);
       break;
     case KVSSD_DTYPE_F32:
-      launch_merge_typed(parts, splits, query_heads, head_dim, static_cast<float*>(out), lse, stream);
+      launch_merge_as<float>(parts, splits, noted, query_heads, head_dim, out, lse, stream);
       break;
     case KVSSD_DTYPE_F64:
-      launch_merge_typed(parts, splits, query_heads, head_dim, static_cast<double*>(out), lse, stream);
+      launch_merge_as<double>(parts, splits, noted, query_heads, head_dim, out, lse, stream);
       break;
     default:
       return arg_error("unsupported output dtype");

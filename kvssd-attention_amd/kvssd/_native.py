@@ -71,6 +71,7 @@ SIGNATURES = {
     "kvssd_hip_abi_version": (_I, []),
     "kvssd_hip_build_id": (ctypes.c_char_p, []),
     "kvssd_hip_device_ok": (_I, [_I, ctypes.c_char_p, _SZ]),
+    "kvssd_hip_decode_plan": (_I, [ctypes.POINTER(DecodeDesc)] + [_VP] * 4 + [ctypes.POINTER(_I)] * 3),
     "kvssd_hip_decode_workspace_bytes": (_I, [ctypes.POINTER(DecodeDesc), ctypes.POINTER(_SZ)]),
     "kvssd_hip_decode_kernel": (_I, [ctypes.POINTER(DecodeDesc), ctypes.POINTER(_I)]),
     "kvssd_hip_fused_decode": (_I, [ctypes.POINTER(DecodeDesc)] + [_VP] * 10 + [_SZ, _VP]),

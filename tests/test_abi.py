@@ -112,6 +112,45 @@ def test_kernel_choice_is_reported():
     assert lib.kvssd_hip_decode_kernel(ctypes.byref(desc), ctypes.byref(k)) == 0
 
 
+def decode_plan(desc, address):
+    kernel, tiled, splits = ctypes.c_int(-1), ctypes.c_int(-1), ctypes.c_int(-1)
+    rc = _native.load().kvssd_hip_decode_plan(ctypes.byref(desc), *[ctypes.c_void_p(address)] * 4, ctypes.byref(kernel),
+                                              ctypes.byref(tiled), ctypes.byref(splits))
+    assert rc == 0, _native.last_error()
+    return kernel.value, tiled.value, splits.value
+
+
+@pytest.mark.parametrize(("shape", "tile_splits", "most"), [
+    # query heads, kv heads, head_dim, blocks, block_tokens, bits, group size, dtype
+    ((64, 4, 256, 256, 64, 4, 16, 2), 8, 256),     # 16K tokens, fp32, GQA 16
+    ((24, 4, 256, 385, 64, 4, 64, 1), 49, 193),    # 24K tokens, bf16, GQA 6
+    ((4, 1, 128, 13, 16, 4, 32, 0), 1, 13),        # 200 tokens, one kv head
+])
+def test_the_split_plan_is_the_running_kernels(shape, tile_splits, most):
+    # arrays that the tiled kernel cannot load go to the vector kernel with that kernel's own,
+    # finer splits (it walks its blocks one after another)
+    desc = _native.DecodeDesc(*shape, 0, 0, 0.1)
+    assert decode_plan(desc, 4096) == (_native.KERNEL_GENERAL, 1, tile_splits)
+    for address in (4096 + 8, 4096 + 4):
+        assert decode_plan(desc, address) == (_native.KERNEL_GENERAL, 0, most)
+    n = ctypes.c_size_t(0)
+    assert _native.load().kvssd_hip_decode_workspace_bytes(ctypes.byref(desc), ctypes.byref(n)) == 0
+    assert n.value >= 4 * most * shape[0] * (shape[2] + 2)
+
+
+def test_the_plan_follows_the_arrays_alignment():
+    # a matrix-core shape: staged on 16-byte boundaries, vector kernel 4 bytes off, an error where
+    # the staged kernel is asked for by name
+    desc = _native.DecodeDesc(32, 8, 128, 1024, 128, 4, 32, 0, 0, 0, 0.1)
+    kernel, tiled, splits = decode_plan(desc, 4096)
+    assert (kernel, tiled) == (_native.KERNEL_STAGED, 0)
+    assert decode_plan(desc, 4096 + 4) == (_native.KERNEL_GENERAL, 0, splits)
+    desc.kernel = _native.KERNEL_STAGED
+    out = [ctypes.byref(ctypes.c_int(0)) for _ in range(3)]
+    assert _native.load().kvssd_hip_decode_plan(ctypes.byref(desc), *[ctypes.c_void_p(4104)] * 4, *out) < 0
+    assert "16-byte aligned" in _native.last_error()
+
+
 def test_record_codec_sizes_and_argument_errors():
     # sizes and argument checks of the record and vLLM codecs need no GPU
     lib = _native.load()

@@ -11,12 +11,14 @@ tolerance for its interpreted kernel.
 
 from __future__ import annotations
 
+import ctypes
 import math
 
 import numpy as np
 import pytest
 import torch
 
+from kvssd import _native
 from kvssd.backends import PackedBatch
 from kvssd.backends.hip import HipAttentionBackend
 from oracle import oracle as O
@@ -87,9 +89,54 @@ def test_tile_edges(cuda_device, bits, qh, kvh, d, g, bt, nb, dtype, selected):
     size = max(1.0, float(np.abs(ref_out).max()))
     for name, args in (("tile", arrays), ("vector", [offset_copy(a, 8) for a in arrays])):
         batch = PackedBatch(*args, counts, bits, g)
+        tiled, _ = split_plan(backend.describe(query, batch, scale, 0 if table is None else len(table)), args)
+        assert tiled == (name == "tile")
         out, lse = backend.run(query, batch, scale, block_table=None if table is None else table.tolist())
         np.testing.assert_allclose(out.cpu().numpy(), ref_out, atol=TOL * size, rtol=TOL, err_msg=name)
         np.testing.assert_allclose(lse.cpu().numpy(), ref_lse, atol=TOL, rtol=TOL, err_msg=name)
+
+
+def split_plan(desc, arrays) -> tuple[int, int]:
+    """(1 where the tiled kernel runs and 0 where the vector one does, splits) of a decode of these arrays."""
+    kernel, tiled, splits = ctypes.c_int(-1), ctypes.c_int(-1), ctypes.c_int(-1)
+    rc = _native.load().kvssd_hip_decode_plan(
+        ctypes.byref(desc), *[t.data_ptr() for t in arrays], ctypes.byref(kernel), ctypes.byref(tiled), ctypes.byref(splits)
+    )
+    assert rc == 0 and kernel.value == _native.KERNEL_GENERAL
+    return tiled.value, splits.value
+
+
+# shapes whose tiled form takes fewer splits than the vector one, and the same number
+@pytest.mark.parametrize(("bits", "qh", "kvh", "d", "g", "bt", "nb"), [(4, 4, 1, 128, 32, 16, 67), (4, 32, 2, 256, 16, 64, 150),
+                                                                         (2, 12, 2, 64, 32, 32, 40), (4, 16, 8, 128, 64, 128, 9)])
+def test_two_phase_calls(cuda_device, bits, qh, kvh, d, g, bt, nb):
+    # partials and merge as separate calls, of arrays that the tiled kernel takes and of such that
+    # it does not: the merge has no arrays to tell by, and finds the number of splits in the partials
+    gen = torch.Generator(device=cuda_device).manual_seed(d + nb)
+    packed = [torch.randint(0, 256, (nb, bt, kvh, d * bits // 8), dtype=torch.uint8, generator=gen, device=cuda_device) for _ in "kv"]
+    scales = [torch.rand(nb, bt, kvh, d // g, generator=gen, device=cuda_device).half() / 8 for _ in "kv"]
+    counts = torch.full((nb,), bt, dtype=torch.int32, device=cuda_device)
+    counts[-1] = 3
+    query = torch.randn(qh, d, generator=gen, device=cuda_device)
+    backend, lib = HipAttentionBackend("auto"), _native.load()
+    stream = _native.stream_handle(torch.cuda.current_stream(cuda_device))
+    plans = []
+    for by in (0, 8):
+        arrays = [offset_copy(t, by) for t in (*packed, *scales)]
+        batch = PackedBatch(*arrays, counts, bits, g)
+        want, want_lse = backend.run(query, batch, 0.1)
+        desc = backend.describe(query, batch, 0.1)
+        plans.append(split_plan(desc, arrays))
+        need = ctypes.c_size_t(0)
+        _native.check(lib.kvssd_hip_decode_workspace_bytes(ctypes.byref(desc), ctypes.byref(need)), "workspace")
+        work = torch.full((need.value,), 255, dtype=torch.uint8, device=cuda_device)  # NaN where nothing is written
+        out, lse = torch.empty_like(want), torch.empty_like(want_lse)
+        args = [t.data_ptr() for t in (query, *arrays, counts)]
+        _native.check(lib.kvssd_hip_decode_partials(ctypes.byref(desc), *args, None, work.data_ptr(), need.value, stream), "partials")
+        _native.check(lib.kvssd_hip_decode_merge(ctypes.byref(desc), work.data_ptr(), need.value, out.data_ptr(), lse.data_ptr(), stream), "merge")
+        torch.testing.assert_close(out, want, atol=TOL, rtol=TOL)
+        torch.testing.assert_close(lse, want_lse, atol=TOL, rtol=TOL)
+    assert [tiled for tiled, _ in plans] == [1, 0] and plans[0][1] <= plans[1][1]
 
 
 @pytest.mark.parametrize("d", [64, 128, 256])
