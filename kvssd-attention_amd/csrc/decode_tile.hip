@@ -10,9 +10,10 @@
 //
 // Measured against the vector kernel on the same arrays (fp16 queries, split
 // and merge): 32K tokens in 32-token blocks, 8 kv heads, GQA 4, head_dim 128
-// 372 -> 15.9 us (37.7 MB of codes and scales); 24K tokens, 4 kv heads, GQA 6,
-// head_dim 256, groups of 64, bf16 222 -> 21.4 us; 16K tokens, head_dim 64 (the
-// kernel alone) 60 -> 10 us.  Output error against float64 0.5-1.2 times its.
+// 372 -> 16.3 us (37.7 MB of codes and scales); 24K tokens, 4 kv heads, GQA 6,
+// head_dim 256, groups of 64, bf16 222 -> 21.3 us; 16K tokens, head_dim 64 (the
+// kernel alone) 60 -> 10 us.  Output error against float64 (rms over 192 to 1,600
+// heads of a shape): INT4 0.53-0.89 times the vector kernel's, INT2 0.82-1.08.
 // What bounds it now: ~5 us of a workgroup's start and end (argument, table and
 // query round trips, the waves' merge), and in between its 64-byte pieces of
 // rows, which HBM serves at ~4 TB/s.
@@ -24,14 +25,17 @@
 // waves' states meet in LDS at the end, one partial per query head.
 //
 // QK (v_mfma_f32_16x16x32_f16): A = query, row r = (head, group) holding that
-//   head masked to that group; B = the codes of 16 tokens, lane (li, lq) the
+//   head masked to that group, scaled by a power of two of its own; B = the codes of 16 tokens, lane (li, lq) the
 //   lq-th quarter of token li's row.  Lane (li, lq) ends with rows 4 lq ..
 //   4 lq + 3 of token li, applies each row's K scale and adds the groups of a
 //   head: in registers up to 4 groups, across lane rows beyond.
-// Softmax: running (m, l) in log2 units per lane row and head.  The weights
-//   W = 2^(s - m) 2^k scale_v carry a whole exponent k that follows the largest
-//   score + V-scale exponent seen, so the largest W lies in [2^12, 2^14)
-//   whatever the scales and both its fp16 parts are normal numbers.
+// Softmax: running (m, l) in log2 units per lane row and head, m a whole number,
+//   so that every rescaling is exact.  The weights W = 2^(s - m) scale_v 2^k carry
+//   a whole exponent k per row (head, group) that follows the row's largest, so
+//   that one lies in [2^12, 2^13) whatever the scales, and W, as two fp16 parts,
+//   is off by at most 2^-23 of itself or 2^-37 of the row's largest.  (One k for a
+//   head's groups left a group of V scales 2^-18 times the head's largest with 8
+//   times the vector kernel's error.)
 // PV: A = W (rows (head, group), K = 32 tokens, hi and lo parts through LDS),
 //   B = V codes from a nibble transpose read (ds_read_b64_tr_b4) of the rows
 //   staged in LDS.  Of a column (dim), the rows of its own group count.
@@ -292,17 +296,24 @@ __device__ __forceinline__ void load_pass(TileLoads<BITS, D, HS>& ld, const Tile
   }
 }
 
-// Per lane row and head: (m, l), the largest score + V-scale exponent so far
-// and the exponent k the accumulators carry; the accumulators
+// Per lane row and head (m, l); per row the exponent k that its accumulators carry
 template <int NT, int HS>
 struct TileState {
-  float m[HS], l[HS], w[HS], k[HS];
+  float m[HS], l[HS];
+  int k[4];
   f32x4 acc[NT];
 };
+constexpr int kMostExponent = 123;  // 2^k and 2^-k are normal numbers; weights below 2^-110 lose bits
+constexpr int kFar = -1000;         // an exponent that ldexpf turns any finite value into 0 by
+
+// m - to as a whole number, m <= to whole (kFar where they are infinite)
+__device__ __forceinline__ int whole_diff(float m, float to) {
+  return static_cast<int>(fmaxf(m - to, static_cast<float>(kFar)));
+}
 
 template <int BITS, int D, int HS, int QSPLIT>
 __device__ __forceinline__ void tile_pass(const TileLoads<BITS, D, HS>& ld, uint8_t* v_lds, uint8_t* w_lds,
-                                          const uint8_t* q_lds, const float (&kscale)[HS],
+                                          const uint8_t* q_lds, const float* q_scale, float scale_log2,
                                           TileState<TileGeo<BITS, D, HS>::NT, HS>& st, int group_shift, int li,
                                           int lq, uint32_t oz) {
   using G = TileGeo<BITS, D, HS, QSPLIT>;
@@ -351,15 +362,19 @@ __device__ __forceinline__ void tile_pass(const TileLoads<BITS, D, HS>& ld, uint
     }
     __builtin_amdgcn_sched_barrier(0);  // (unpacking further ahead costs registers, i.e. resident waves)
   }
+  const f32x4 row_scale = *reinterpret_cast<const f32x4*>(q_scale + 4 * lq);  // of this lane's query rows
 #pragma unroll
   for (int tau = 0; tau < 4; ++tau) {
     if constexpr (QSPLIT > 1) c[tau] += rest[tau];
 #pragma unroll
     for (int hs = 0; hs < HS; ++hs) {
-      float s = half_bits_to_float(scale_bits(ld.sk[tau], 0)) * c[tau][hs * NG];
+      float s = 0.0f;
 #pragma unroll
-      for (int i = 1; i < NG; ++i)
-        s = __builtin_fmaf(half_bits_to_float(scale_bits(ld.sk[tau], i)), c[tau][hs * NG + i], s);
+      for (int i = 0; i < NG; ++i) {
+        const float k = half_bits_to_float(scale_bits(ld.sk[tau], i));
+        const float ci = c[tau][hs * NG + i] * row_scale[hs * NG + i];  // (a power of two: exact)
+        s = i == 0 ? k * ci : __builtin_fmaf(k, ci, s);
+      }
       score[hs][tau] = s;
     }
     if constexpr (HS == 1) {  // 8 or 16 groups: a head's rows lie in 2 or 4 lane rows
@@ -369,77 +384,65 @@ __device__ __forceinline__ void tile_pass(const TileLoads<BITS, D, HS>& ld, uint
   }
   // --------------------------------------------------------------- softmax
   float sv[4][NG];  // V scales, 0 for masked tokens (a stale scale may not be finite)
-  float e_v[4];
   bool ok[4];
 #pragma unroll
   for (int tau = 0; tau < 4; ++tau) {
     ok[tau] = (ld.ok >> tau) & 1u;
-    uint32_t big = 0u;
 #pragma unroll
-    for (int i = 0; i < NG; ++i) {
-      const uint16_t h = ok[tau] ? scale_bits(ld.sv[tau], i) : static_cast<uint16_t>(0);
-      sv[tau][i] = half_bits_to_float(h);
-      big = max(big, static_cast<uint32_t>(h) & 0x7FFFu);
-    }
-    // exponent of the largest |scale| (a zero or subnormal one counts as 2^-14)
-    e_v[tau] = static_cast<float>(max(static_cast<int>(big >> 10), 1) - 15);
-  }
-  float pk[HS][4];    // p 2^k
-  float alpha[HS];    // what the accumulators so far count relative to the new references
-  bool rescale = false;
-#pragma unroll
-  for (int hs = 0; hs < HS; ++hs) {
-    float sc[4], mx = -INFINITY, wx = -INFINITY;
-#pragma unroll
-    for (int tau = 0; tau < 4; ++tau) {
-      sc[tau] = ok[tau] ? score[hs][tau] * kscale[hs] : -INFINITY;
-      mx = fmaxf(mx, sc[tau]);
-      wx = fmaxf(wx, sc[tau] + e_v[tau]);
-    }
-    const float m_new = fmaxf(st.m[hs], row_max16(mx));
-    const float w_new = fmaxf(st.w[hs], row_max16(wx));
-    const bool none = m_new == -INFINITY;
-    const float m_use = none ? 0.0f : m_new;
-    // a whole number, so that p 2^k is as exact as p: w_new - m_new lies in [-14, 16]
-    const float k_new = none ? 0.0f : 13.0f - ceilf(w_new - m_use);
-    const float a_l = none ? 1.0f : __builtin_amdgcn_exp2f(st.m[hs] - m_use);
-    alpha[hs] = a_l * __builtin_amdgcn_exp2f(k_new - st.k[hs]);
-    st.m[hs] = m_new;
-    st.w[hs] = w_new;
-    st.k[hs] = k_new;
-    rescale = rescale || alpha[hs] != 1.0f;
-    const float two_k = __builtin_amdgcn_exp2f(k_new);
-    float sum = 0.0f;
-#pragma unroll
-    for (int tau = 0; tau < 4; ++tau) {
-      const float pr = __builtin_amdgcn_exp2f(sc[tau] - m_use);
-      sum += pr;
-      pk[hs][tau] = pr * two_k;
-    }
-    st.l[hs] = __builtin_fmaf(st.l[hs], a_l, sum);
+    for (int i = 0; i < NG; ++i) sv[tau][i] = half_bits_to_float(ok[tau] ? scale_bits(ld.sv[tau], i) : static_cast<uint16_t>(0));
   }
   // W rows 4 lq + i: this lane's four tokens in slots 4 u .. 4 u + 3
   const int u = 8 * ((li >> 1) & 1) + 2 * (li >> 2) + (li & 1);
+  int shift[4];  // log2 of what the accumulators so far count relative to the new references
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int hs = i / NG, gi = i % NG;
-    u32x2 hi, lo;
-    uint32_t h, l;
-    split_pair(pk[hs][0] * sv[0][gi], pk[hs][1] * sv[1][gi], h, l);
-    hi[0] = h;
-    lo[0] = l;
-    split_pair(pk[hs][2] * sv[2][gi], pk[hs][3] * sv[3][gi], h, l);
-    hi[1] = h;
-    lo[1] = l;
-    uint8_t* dst = w_lds + (4 * lq + i) * kWRowBytes + 8 * u;
-    *reinterpret_cast<u32x2*>(dst) = hi;
-    *reinterpret_cast<u32x2*>(dst + 16 * kWRowBytes) = lo;
+  for (int hs = 0; hs < HS; ++hs) {
+    float sc[4], mx = -INFINITY;
+#pragma unroll
+    for (int tau = 0; tau < 4; ++tau) {
+      sc[tau] = ok[tau] ? score[hs][tau] * scale_log2 : -INFINITY;
+      mx = fmaxf(mx, sc[tau]);
+    }
+    const float m_new = fmaxf(st.m[hs], ceilf(row_max16(mx)));
+    const float m_use = m_new == -INFINITY ? 0.0f : m_new;
+    const int dm = whole_diff(st.m[hs], m_use);
+    st.m[hs] = m_new;
+    float sum = 0.0f;
+#pragma unroll
+    for (int tau = 0; tau < 4; ++tau) {
+      sc[tau] = __builtin_amdgcn_exp2f(sc[tau] - m_use);
+      sum += sc[tau];
+    }
+    st.l[hs] = ldexpf(st.l[hs], dm) + sum;
+#pragma unroll
+    for (int gi = 0; gi < NG; ++gi) {
+      const int i = hs * NG + gi;
+      float w[4];
+#pragma unroll
+      for (int tau = 0; tau < 4; ++tau) w[tau] = sc[tau] * sv[tau][gi];
+      const float big = row_max16(fmaxf(fmaxf(fabsf(w[0]), fabsf(w[1])), fmaxf(fabsf(w[2]), fabsf(w[3]))));
+      // (big in [2^(e - 1), 2^e), e its frexp exponent)
+      const int most = big > 0.0f ? 13 - __builtin_amdgcn_frexp_expf(big) : kMostExponent;
+      const int k = min(min(st.k[i] - dm, most), kMostExponent);
+      shift[i] = dm + k - st.k[i];
+      st.k[i] = k;
+      u32x2 hi, lo;
+      uint32_t h, l;
+      split_pair(ldexpf(w[0], k), ldexpf(w[1], k), h, l);
+      hi[0] = h;
+      lo[0] = l;
+      split_pair(ldexpf(w[2], k), ldexpf(w[3], k), h, l);
+      hi[1] = h;
+      lo[1] = l;
+      uint8_t* dst = w_lds + (4 * lq + i) * kWRowBytes + 8 * u;
+      *reinterpret_cast<u32x2*>(dst) = hi;
+      *reinterpret_cast<u32x2*>(dst + 16 * kWRowBytes) = lo;
+    }
   }
-  if (__any(rescale)) {
+  if (__any((shift[0] | shift[1] | shift[2] | shift[3]) != 0)) {
 #pragma unroll
     for (int n = 0; n < G::NT; ++n)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) st.acc[n][i] *= alpha[i / NG];
+      for (int i = 0; i < 4; ++i) st.acc[n][i] = ldexpf(st.acc[n][i], shift[i]);
   }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -473,6 +476,58 @@ __device__ __forceinline__ void tile_pass(const TileLoads<BITS, D, HS>& ld, uint
   __builtin_amdgcn_wave_barrier();  // the next pass's LDS writes stay behind these reads
 }
 
+// v[e], of dim lane + 64 e of a head, becomes the largest of v >= 0 over the
+// dim's group `own` (HS == 4: over the head).  Without branches, under which the pass's loads in flight
+// would cost registers, where head_dim is a power of two.  `scratch`: an LDS
+// word a group, the wave's own.
+template <int D, int HS, int QE>
+__device__ __forceinline__ void group_max(float (&v)[QE], const int (&own)[QE], int* scratch, int group_size) {
+  const int lane = threadIdx.x & (kWave - 1);
+  if constexpr (HS == 4) {
+    float m = v[0];
+#pragma unroll
+    for (int e = 1; e < QE; ++e) m = fmaxf(m, v[e]);
+    m = wave_max(m);
+#pragma unroll
+    for (int e = 0; e < QE; ++e) v[e] = m;
+  } else if constexpr (HS == 2 && D % 128 == 0) {  // two groups of whole waves
+    constexpr int kPer = QE / 2;
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      float m = v[g * kPer];
+#pragma unroll
+      for (int e = 1; e < kPer; ++e) m = fmaxf(m, v[g * kPer + e]);
+      m = wave_max(m);
+#pragma unroll
+      for (int e = 0; e < kPer; ++e) v[g * kPer + e] = m;
+    }
+  } else if (D % kWave == 0 || (group_size & (group_size - 1)) == 0) {  // runs of 4 to 64 lanes, a power of two
+#pragma unroll
+    for (int e = 0; e < QE; ++e) {
+      float m = fmaxf(v[e], quad_lane<0xB1>(v[e]));
+      m = fmaxf(m, quad_lane<0x4E>(m));
+      const float m8 = fmaxf(m, quad_lane<0x141>(m));  // with the other quad of 8
+      m = group_size > 4 ? m8 : m;
+      const float m16 = fmaxf(m, quad_lane<0x140>(m));  // with the other half of 16
+      m = group_size > 8 ? m16 : m;
+      const float m01 = fmaxf(lane_value(m, 0), lane_value(m, 16)), m23 = fmaxf(lane_value(m, 32), lane_value(m, 48));
+      v[e] = group_size > 32 ? fmaxf(m01, m23) : group_size > 16 ? (lane < 32 ? m01 : m23) : m;
+    }
+  } else {  // head_dim 96 in other groups: the largest bits (lanes past the row's end repeat its last value)
+    const int groups = D / group_size;
+    if (lane < groups) scratch[lane] = 0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int e = 0; e < QE; ++e)
+      __hip_atomic_fetch_max(scratch + own[e], __builtin_bit_cast(int, v[e]), __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_WORKGROUP);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int e = 0; e < QE; ++e) v[e] = __builtin_bit_cast(float, scratch[own[e]]);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+}
+
 template <int BITS, int D, int HS, int QSPLIT>
 __global__ __launch_bounds__(kTileThreads, tile_workgroups_per_cu(D, HS, QSPLIT)) void decode_tile_kernel(
     const void* query, const uint8_t* pk, const uint8_t* pv, const uint16_t* sk, const uint16_t* sv, uint32_t shape,
@@ -481,7 +536,7 @@ __global__ __launch_bounds__(kTileThreads, tile_workgroups_per_cu(D, HS, QSPLIT)
   constexpr int NG = G::NG;
   __shared__ __attribute__((aligned(16))) uint8_t lds[G::LDS];
   __shared__ __attribute__((aligned(16))) float ml[4][HS][2][kTileWaves];  // [lane row][head][m, l][wave]
-  __shared__ int q_exp[G::HEADS];
+  __shared__ __attribute__((aligned(16))) float q_scale[16];  // what a query row's operand counts by
   const TileParams p{pk, pv, sk, sv, static_cast<int>(shape & 0xFFFFu), static_cast<int>((shape >> 16) & 0x1Fu),
                      static_cast<int>((shape >> 21) & 7u), block_tokens, (shape & kHasTable) != 0};
 
@@ -549,52 +604,56 @@ __global__ __launch_bounds__(kTileThreads, tile_workgroups_per_cu(D, HS, QSPLIT)
   // ------------------------------------------------------------------ query
   // A operand rows (head, group) in LDS, in K-slot order: a head's values in
   // the row of their group, zeros in its other rows.  Values are scaled by
-  // 2^(14 - ex), ex the exponent of the head's largest, so that every part of
-  // all but negligible values is a normal fp16.
+  // 2^(kTop - ex), ex the exponent of the largest: over the head for 16-bit
+  // queries, of which one part holds fp16 values exactly and bf16 values down to
+  // 2^-32 of the largest (below, to 2^-40 of it); over the row for the three
+  // parts of wider ones, which leave at most 2^-39 of the row's largest.  (Rows
+  // for all of them: 0.4-0.8 us of 17-22.)
+  constexpr int kTop = QSPLIT == 1 ? 15 : 14;
+  const int group_size = D % kWave == 0 ? D >> group_shift : D / p.groups;
   uint8_t* q_lds = lds + G::Q_OFF;
 #pragma unroll
   for (int i = 0; i < HS; ++i) {
     const int h = wave + kTileWaves * i;
     if (h >= (16 >> group_shift)) break;
-    float mx = 0.0f;
+    int own[QE];
+    float mx[QE];
 #pragma unroll
     for (int e = 0; e < QE; ++e) {
+      own[e] = static_cast<int>((static_cast<uint32_t>(min(lane + kWave * e, D - 1)) * r.group_magic) >> 16);
       if (h >= nh) qx[i][e] = 0.0f;
-      mx = fmaxf(mx, fabsf(qx[i][e]));
+      const float x = fabsf(qx[i][e]);
+      mx[e] = x < INFINITY ? x : 0.0f;
     }
-    mx = wave_max(mx);
-    const int ex = mx > 0.0f && mx < INFINITY ? __builtin_amdgcn_frexp_expf(mx) - 1 : 0;  // mx in [2^ex, 2^(ex + 1))
-    if (lane == 0) q_exp[h] = ex;
+    group_max<D, QSPLIT == 1 ? 4 : HS>(mx, own, reinterpret_cast<int*>(q_scale) + (h << group_shift), group_size);
 #pragma unroll
     for (int e = 0; e < QE; ++e) {
       const int d = lane + kWave * e;
       if (D % kWave != 0 && d >= D) break;
-      float rem = ldexpf(qx[i][e], 14 - ex);
+      const int ex = (mx[e] > 0.0f ? __builtin_amdgcn_frexp_expf(mx[e]) - 1 : 0) - kTop;  // mx in [2^ex, 2^(ex + 1))
+      q_scale[(h << group_shift) + own[e]] = ldexpf(1.0f, ex);
+      float rem = ldexpf(qx[i][e], -ex);
       _Float16 part[QSPLIT];
 #pragma unroll
       for (int sp = 0; sp < QSPLIT; ++sp) {
         part[sp] = static_cast<_Float16>(rem);
         rem = fmaxf(rem - static_cast<float>(part[sp]), -65504.0f);
       }
-      const int own = static_cast<int>((static_cast<uint32_t>(d) * r.group_magic) >> 16);
       uint8_t* dst = q_lds + (h << group_shift) * G::Q_ROW + 2 * query_slot<BITS, D>(d);
       for (int g = 0; g < (1 << group_shift); ++g, dst += G::Q_ROW)
 #pragma unroll
         for (int sp = 0; sp < QSPLIT; ++sp)
-          *reinterpret_cast<_Float16*>(dst + 16 * sp * G::Q_ROW) = g == own ? part[sp] : static_cast<_Float16>(0.0f);
+          *reinterpret_cast<_Float16*>(dst + 16 * sp * G::Q_ROW) = g == own[e] ? part[sp] : static_cast<_Float16>(0.0f);
     }
   }
   __syncthreads();
-  float kscale[HS];
   TileState<G::NT, HS> st;
 #pragma unroll
+  for (int i = 0; i < 4; ++i) st.k[i] = kMostExponent;
+#pragma unroll
   for (int hs = 0; hs < HS; ++hs) {
-    const int h = HS == 1 ? lq >> span_shift : HS * lq + hs;
-    kscale[hs] = ldexpf(r.scale_log2, q_exp[h] - 14);
     st.m[hs] = -INFINITY;
     st.l[hs] = 0.0f;
-    st.w[hs] = -INFINITY;
-    st.k[hs] = 0.0f;
   }
 #pragma unroll
   for (int n = 0; n < G::NT; ++n) st.acc[n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -605,7 +664,7 @@ __global__ __launch_bounds__(kTileThreads, tile_workgroups_per_cu(D, HS, QSPLIT)
   uint8_t* v_lds = lds + wave * G::WAVE_BYTES;
   uint8_t* w_lds = v_lds + G::V_BYTES;
   while (have) {
-    tile_pass<BITS, D, HS, QSPLIT>(ld, v_lds, w_lds, q_lds, kscale, st, group_shift, li, lq, oz);
+    tile_pass<BITS, D, HS, QSPLIT>(ld, v_lds, w_lds, q_lds, q_scale, r.scale_log2, st, group_shift, li, lq, oz);
     base_off += kTileThreads;  // (64 slots per wave and pass)
     const uint32_t q = ((base_off * r.bt_magic) >> 20) + (bt >= 256u && base_off >= bt ? 1u : 0u);
     base_unit += static_cast<int>(q);
@@ -627,7 +686,7 @@ __global__ __launch_bounds__(kTileThreads, tile_workgroups_per_cu(D, HS, QSPLIT)
   __syncthreads();  // (m, l) of every wave; every V, W and query region is free
   const int span = 1 << span_shift;
   // the largest m of a head: over the waves and its lane rows, whose m differ
-  // in nothing but rounding
+  // by a rounding (and so at most by one, past a whole number)
   auto head_max = [&](int row, int hs) {
     float big = -INFINITY;
     for (int i = 0; i < span; ++i) {
@@ -642,7 +701,7 @@ __global__ __launch_bounds__(kTileThreads, tile_workgroups_per_cu(D, HS, QSPLIT)
     const int h = HS == 1 ? lq >> span_shift : HS * lq + hs;
     const float big = head_max(lq & ~(span - 1), hs);
     const bool some = ml[lq][hs][1][wave] != 0.0f;
-    const float back = some ? __builtin_amdgcn_exp2f(st.m[hs] - big) * __builtin_amdgcn_exp2f(-st.k[hs]) : 0.0f;
+    const int dm = whole_diff(st.m[hs], big);
     if (h < nh) {
       float* xrow = xo + (wave * G::HEADS + h) * D;
 #pragma unroll
@@ -653,14 +712,14 @@ __global__ __launch_bounds__(kTileThreads, tile_workgroups_per_cu(D, HS, QSPLIT)
           const int gt = static_cast<int>((static_cast<uint32_t>(dim) * r.group_magic) >> 16);
           const f32x4 a = st.acc[G::NPAR * n + par];
           float o = a[hs * NG];
-          if constexpr (NG == 2) o = (gt & 1) ? a[hs * NG + 1] : o;
-          if constexpr (NG == 4) {
-            o = (gt & 3) == 1 ? a[1] : o;
-            o = (gt & 3) == 2 ? a[2] : o;
-            o = (gt & 3) == 3 ? a[3] : o;
+          int k = st.k[hs * NG];
+#pragma unroll
+          for (int i = 1; i < NG; ++i) {
+            o = (gt & (NG - 1)) == i ? a[hs * NG + i] : o;
+            k = (gt & (NG - 1)) == i ? st.k[hs * NG + i] : k;
           }
           const bool mine = NG < 4 || (gt >> 2) == (lq & (span - 1));
-          if (mine) xrow[dim] = some ? o * back : 0.0f;
+          if (mine) xrow[dim] = some ? ldexpf(o, dm - k) : 0.0f;
         }
     }
   }

@@ -96,6 +96,61 @@ def test_tile_edges(cuda_device, bits, qh, kvh, d, g, bt, nb, dtype, selected):
         np.testing.assert_allclose(lse.cpu().numpy(), ref_lse, atol=TOL, rtol=TOL, err_msg=name)
 
 
+# bits, query heads, kv heads, head_dim, group size, query dtype: 2, 4, 6, 8 and 16 groups a head
+GROUPED = [(4, 8, 2, 128, 64, torch.float32), (4, 8, 2, 64, 16, torch.float16), (4, 6, 2, 96, 16, torch.bfloat16),
+           (2, 4, 1, 256, 32, torch.float32), (4, 4, 4, 128, 8, torch.float32), (4, 4, 2, 96, 48, torch.float32)]
+
+
+def grouped_case(rng, bits, kvh, d, g, spread):
+    """Keys or values of 9 blocks of 48 tokens whose first group is 2^spread times the size of the others."""
+    x = rng.standard_normal((9 * 48, kvh, d)).astype(np.float32) * np.float32(2.0 ** (-spread / 2))
+    x[..., :g] *= np.float32(2.0 ** spread)
+    packed, scales, valid = O.quantize_blocks(x, bits, g, 48)
+    return packed, scales, valid
+
+
+@pytest.mark.parametrize(("bits", "qh", "kvh", "d", "g", "dtype"), GROUPED)
+@pytest.mark.parametrize("spread", [-22, 22])
+def test_value_groups_far_apart(cuda_device, bits, qh, kvh, d, g, dtype, spread):
+    # a value group whose scales lie 2^-22 below (or above) the other groups' is as exact as those,
+    # compared by itself.  A weight is off by one rounding of p scale_v, one of p (scores below 8:
+    # ~2^-21 at most) and 2^-23 of its two parts, some 1e-6 together in the worst case
+    rng = np.random.default_rng(d + g)
+    pk, sk, valid = grouped_case(rng, bits, kvh, d, g, 0)
+    pv, sv, _ = grouped_case(rng, bits, kvh, d, g, spread)
+    q = torch.from_numpy(rng.standard_normal((qh, d)).astype(np.float32)).to(dtype)
+    ref, _ = O.attention(q.float().numpy(), pk, pv, sk, sv, valid, bits, g, 1 / math.sqrt(d))
+    arrays = [torch.from_numpy(a).to(cuda_device) for a in (pk, pv, sk, sv)]
+    batch = PackedBatch(*arrays, torch.from_numpy(valid).to(cuda_device), bits, g)
+    backend = HipAttentionBackend("auto")
+    assert split_plan(backend.describe(q.to(cuda_device), batch, 1.0), arrays)[0] == 1
+    out, _ = backend.run(q.to(cuda_device), batch, 1 / math.sqrt(d))
+    err = (out.double().cpu().numpy() - ref).reshape(qh, -1, g)
+    size = np.asarray(ref, dtype=np.float64).reshape(qh, -1, g)
+    assert (np.linalg.norm(err, axis=(0, 2)) < 2e-6 * np.linalg.norm(size, axis=(0, 2))).all()
+
+
+@pytest.mark.parametrize(("bits", "qh", "kvh", "d", "g", "dtype"), GROUPED)
+def test_query_groups_far_apart(cuda_device, bits, qh, kvh, d, g, dtype):
+    # a query group 2^-26 below the others counts as much as they do where its keys lie 2^26 above
+    # them: a score (below 16 here) is then as exact as any, some ten roundings of 2^-24 of it
+    if dtype == torch.float16:
+        dtype = torch.bfloat16  # (2^-26 of an fp16 query is zero)
+    rng = np.random.default_rng(d + 2 * g)
+    pk, sk, valid = grouped_case(rng, bits, kvh, d, g, 26)
+    pv, sv, _ = grouped_case(rng, bits, kvh, d, g, 0)
+    q = rng.standard_normal((qh, d)).astype(np.float32)
+    q[:, :g] *= np.float32(2.0 ** -26)
+    q = torch.from_numpy(q).to(dtype)
+    scale = 2.0**13 / math.sqrt(d)
+    ref, ref_lse = O.attention(q.float().numpy(), pk, pv, sk, sv, valid, bits, g, scale)
+    arrays = [torch.from_numpy(a).to(cuda_device) for a in (pk, pv, sk, sv)]
+    batch = PackedBatch(*arrays, torch.from_numpy(valid).to(cuda_device), bits, g)
+    out, lse = HipAttentionBackend("auto").run(q.to(cuda_device), batch, scale)
+    np.testing.assert_allclose(lse.cpu().numpy(), ref_lse, atol=1e-5)
+    assert np.linalg.norm(out.double().cpu().numpy() - ref) < 1e-5 * np.linalg.norm(ref)
+
+
 def split_plan(desc, arrays) -> tuple[int, int]:
     """(1 where the tiled kernel runs and 0 where the vector one does, splits) of a decode of these arrays."""
     kernel, tiled, splits = ctypes.c_int(-1), ctypes.c_int(-1), ctypes.c_int(-1)
