@@ -626,6 +626,8 @@ __global__ __launch_bounds__(kTileThreads, tile_workgroups_per_cu(D, HS, QSPLIT)
       mx[e] = x < INFINITY ? x : 0.0f;
     }
     group_max<D, QSPLIT == 1 ? 4 : HS>(mx, own, reinterpret_cast<int*>(q_scale) + (h << group_shift), group_size);
+    // (rows past the last of 3, 6 or 12 groups hold zeros: any finite factor)
+    if (D == 96 && lane < (1 << group_shift)) q_scale[(h << group_shift) + lane] = 1.0f;
 #pragma unroll
     for (int e = 0; e < QE; ++e) {
       const int d = lane + kWave * e;

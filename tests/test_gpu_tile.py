@@ -194,6 +194,32 @@ def test_two_phase_calls(cuda_device, bits, qh, kvh, d, g, bt, nb):
     assert [tiled for tiled, _ in plans] == [1, 0] and plans[0][1] <= plans[1][1]
 
 
+@pytest.mark.parametrize("g", [32, 16, 8])
+def test_leftover_shared_memory(cuda_device, g):
+    # 3, 6 and 12 groups a head leave rows of the query operand over: what earlier workgroups left in
+    # the LDS (here V rows whose dwords are NaN) must not reach their factors
+    gen = torch.Generator(device=cuda_device).manual_seed(g)
+
+    def batch(d, group, fill):
+        nb, bt, kvh = 64, 64, 8
+        packed = [torch.randint(0, 256, (nb, bt, kvh, d // 2), dtype=torch.uint8, generator=gen, device=cuda_device) for _ in "kv"]
+        if fill:
+            packed[1].fill_(255)
+        scales = [torch.rand(nb, bt, kvh, d // group, generator=gen, device=cuda_device).half() / 8 for _ in "kv"]
+        return PackedBatch(*packed, *scales, torch.full((nb,), bt, dtype=torch.int32, device=cuda_device), 4, group)
+
+    backend = HipAttentionBackend("auto")
+    fills = [(torch.randn(32, d, generator=gen, device=cuda_device), batch(d, 64, True)) for d in (64, 128, 256)]
+    query, cases = torch.randn(32, 96, generator=gen, device=cuda_device), batch(96, g, False)
+    want, want_lse = backend.run(query, PackedBatch(*[offset_copy(t, 8) for t in (cases.packed_k, cases.packed_v, cases.scales_k,
+                                 cases.scales_v)], cases.valid_tokens, 4, g), 0.1)
+    for i in range(12):
+        backend.run(*fills[i % 3], 0.1)
+        out, lse = backend.run(query, cases, 0.1)
+        torch.testing.assert_close(out, want, atol=TOL, rtol=TOL)
+        torch.testing.assert_close(lse, want_lse, atol=TOL, rtol=TOL)
+
+
 @pytest.mark.parametrize("d", [64, 128, 256])
 def test_tile_without_a_valid_token(cuda_device, d):
     pk = torch.randint(0, 256, (5, 32, 2, d // 2), dtype=torch.uint8, device=cuda_device)
