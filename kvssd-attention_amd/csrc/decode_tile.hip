@@ -25,10 +25,11 @@
 // waves' states meet in LDS at the end, one partial per query head.
 //
 // QK (v_mfma_f32_16x16x32_f16): A = query, row r = (head, group) holding that
-//   head masked to that group, scaled by a power of two of its own; B = the codes of 16 tokens, lane (li, lq) the
-//   lq-th quarter of token li's row.  Lane (li, lq) ends with rows 4 lq ..
-//   4 lq + 3 of token li, applies each row's K scale and adds the groups of a
-//   head: in registers up to 4 groups, across lane rows beyond.
+//   head masked to that group, scaled by a power of two; B = the codes of 16
+//   tokens, lane (li, lq) the lq-th quarter of token li's row.  Lane (li, lq)
+//   ends with rows 4 lq .. 4 lq + 3 of token li, applies each row's K scale and
+//   adds the groups of a head: in registers up to 4 groups, across lane rows
+//   beyond.
 // Softmax: running (m, l) in log2 units per lane row and head, m a whole number,
 //   so that every rescaling is exact.  The weights W = 2^(s - m) scale_v 2^k carry
 //   a whole exponent k per row (head, group) that follows the row's largest, so
@@ -209,6 +210,12 @@ __device__ __forceinline__ void load_bytes(void* dst, const void* src) {
   __builtin_memcpy(dst, __builtin_assume_aligned(src, kAlign), BYTES);
 }
 
+// head_dim 96: rows past the last of 3, 6 or 12 groups re-read the scales of
+// groups before; their K scales count as zeros (their sums are zeros, and 0
+// times an infinite scale would not be)
+template <int D, int HS>
+constexpr bool kPadRows = D == 96 && HS == 1;
+
 // the scales of a lane's NG groups, from group gbase on
 template <int NG, bool NARROW>
 __device__ __forceinline__ void load_scales(uint32_t* dst, const uint16_t* row, int gbase, int groups, bool wide) {
@@ -219,7 +226,7 @@ __device__ __forceinline__ void load_scales(uint32_t* dst, const uint16_t* row, 
   } else {
     uint16_t h[NG];
 #pragma unroll
-    for (int i = 0; i < NG; ++i) h[i] = row[min(gbase + i, groups - 1)];  // rows past the last group have a zero query
+    for (int i = 0; i < NG; ++i) h[i] = row[min(gbase + i, groups - 1)];
 #pragma unroll
     for (int i = 0; i < NG; i += 2) dst[i >> 1] = h[i] | (static_cast<uint32_t>(h[i + 1]) << 16);
   }
@@ -314,6 +321,7 @@ __device__ __forceinline__ int whole_diff(float m, float to) {
 template <int BITS, int D, int HS, int QSPLIT>
 __device__ __forceinline__ void tile_pass(const TileLoads<BITS, D, HS>& ld, uint8_t* v_lds, uint8_t* w_lds,
                                           const uint8_t* q_lds, const float* q_scale, float scale_log2,
+                                          const uint32_t (&k_mask)[TileLoads<BITS, D, HS>::SW],
                                           TileState<TileGeo<BITS, D, HS>::NT, HS>& st, int group_shift, int li,
                                           int lq, uint32_t oz) {
   using G = TileGeo<BITS, D, HS, QSPLIT>;
@@ -366,12 +374,15 @@ __device__ __forceinline__ void tile_pass(const TileLoads<BITS, D, HS>& ld, uint
 #pragma unroll
   for (int tau = 0; tau < 4; ++tau) {
     if constexpr (QSPLIT > 1) c[tau] += rest[tau];
+    uint32_t sk[TileLoads<BITS, D, HS>::SW];
+#pragma unroll
+    for (int i = 0; i < TileLoads<BITS, D, HS>::SW; ++i) sk[i] = kPadRows<D, HS> ? ld.sk[tau][i] & k_mask[i] : ld.sk[tau][i];
 #pragma unroll
     for (int hs = 0; hs < HS; ++hs) {
       float s = 0.0f;
 #pragma unroll
       for (int i = 0; i < NG; ++i) {
-        const float k = half_bits_to_float(scale_bits(ld.sk[tau], i));
+        const float k = half_bits_to_float(scale_bits(sk, i));
         const float ci = c[tau][hs * NG + i] * row_scale[hs * NG + i];  // (a power of two: exact)
         s = i == 0 ? k * ci : __builtin_fmaf(k, ci, s);
       }
@@ -590,7 +601,11 @@ __global__ __launch_bounds__(kTileThreads, tile_workgroups_per_cu(D, HS, QSPLIT)
   const int span_shift = group_shift > 2 ? group_shift - 2 : 0;  // lane rows per head: 2^span_shift
   const bool wide_scales = D != 96 || p.groups % NG == 0;  // this lane's groups in one aligned load
   int gbase = NG == 4 ? 4 * (lq & ((1 << span_shift) - 1)) : 0;
-  if (wide_scales) gbase = min(gbase, p.groups - NG);  // (rows of groups past the last have a zero query)
+  uint32_t k_mask[TileLoads<BITS, D, HS>::SW];
+#pragma unroll
+  for (int i = 0; i < TileLoads<BITS, D, HS>::SW; ++i)
+    k_mask[i] = (gbase + 2 * i < p.groups ? 0xFFFFu : 0u) | (gbase + 2 * i + 1 < p.groups ? 0xFFFF0000u : 0u);
+  if (wide_scales) gbase = min(gbase, p.groups - NG);
 
   const uint32_t bt = block_tokens;
   int base_unit = 0;
@@ -666,7 +681,7 @@ __global__ __launch_bounds__(kTileThreads, tile_workgroups_per_cu(D, HS, QSPLIT)
   uint8_t* v_lds = lds + wave * G::WAVE_BYTES;
   uint8_t* w_lds = v_lds + G::V_BYTES;
   while (have) {
-    tile_pass<BITS, D, HS, QSPLIT>(ld, v_lds, w_lds, q_lds, q_scale, r.scale_log2, st, group_shift, li, lq, oz);
+    tile_pass<BITS, D, HS, QSPLIT>(ld, v_lds, w_lds, q_lds, q_scale, r.scale_log2, k_mask, st, group_shift, li, lq, oz);
     base_off += kTileThreads;  // (64 slots per wave and pass)
     const uint32_t q = ((base_off * r.bt_magic) >> 20) + (bt >= 256u && base_off >= bt ? 1u : 0u);
     base_unit += static_cast<int>(q);

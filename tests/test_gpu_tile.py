@@ -220,6 +220,31 @@ def test_leftover_shared_memory(cuda_device, g):
         torch.testing.assert_close(lse, want_lse, atol=TOL, rtol=TOL)
 
 
+@pytest.mark.parametrize("g", [96, 48, 32, 24, 16, 12, 8])
+def test_infinite_key_scale(cuda_device, g):
+    # a token whose last group has an infinite K scale, codes below the middle and a positive query:
+    # its score is -inf and its weight 0, whatever the number of groups that share a matrix operand
+    # (3, 6 and 12 leave rows over); the vector kernel gives the same
+    d, bits, kvh, bt, nb = 96, 4, 2, 16, 5
+    rng = np.random.default_rng(g)
+    pk, sk, valid = O.quantize_blocks(rng.standard_normal((nb * bt, kvh, d)).astype(np.float32), bits, g, bt)
+    pv, sv, _ = O.quantize_blocks(rng.standard_normal((nb * bt, kvh, d)).astype(np.float32), bits, g, bt)
+    q = np.abs(rng.standard_normal((6, d))).astype(np.float32)
+    keep = np.ones((nb, bt), dtype=bool)
+    for b, t in ((0, 3), (2, 0), (4, 15)):
+        keep[b, t] = False
+        sk[b, t, :, -1] = np.inf
+        pk[b, t, :, -g // 2 :] = 0x21  # codes 1 and 2 of the group's values: -7 and -6
+    ref, ref_lse = O.attention(q, *(a[keep][None] for a in (pk, pv)), *(a[keep][None] for a in (sk, sv)),
+                               np.array([keep.sum()], dtype=np.int32), bits, g, 0.1)
+    arrays = [torch.from_numpy(a).to(cuda_device) for a in (pk, pv, sk, sv)]
+    counts = torch.from_numpy(valid).to(cuda_device)
+    for args in (arrays, [offset_copy(a, 8) for a in arrays]):
+        out, lse = HipAttentionBackend("auto").run(torch.from_numpy(q).to(cuda_device), PackedBatch(*args, counts, bits, g), 0.1)
+        np.testing.assert_allclose(out.cpu().numpy(), ref, atol=TOL, rtol=TOL)
+        np.testing.assert_allclose(lse.cpu().numpy(), ref_lse, atol=TOL, rtol=TOL)
+
+
 @pytest.mark.parametrize("d", [64, 128, 256])
 def test_tile_without_a_valid_token(cuda_device, d):
     pk = torch.randint(0, 256, (5, 32, 2, d // 2), dtype=torch.uint8, device=cuda_device)
