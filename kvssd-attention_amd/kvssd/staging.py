@@ -57,6 +57,17 @@ _ALIGN = 256
 # take 5.1, 3.3, 3.0 and 2.7 ms (and, at 4, the host 52 us a chunk for its
 # copy, events and launches), reads by the kernel 2.8 ms whatever the chunk.
 _COPY_CHUNK_BYTES = 8 << 20
+# The vector decode kernel takes a half to the whole of the reads' time, which
+# the ring hides behind its copies where a chunk has a (block, kv head) pair for
+# every CU, some bytes, and enough chunks follow each other (32K tokens of 8 kv
+# heads, INT4, GQA 4, copied against read: 24-token blocks, chunks of 1.2 MB, 336
+# pairs 1.82 against 1.50 ms, 3 MB, 832 pairs 1.16 against 1.48; head_dim 112, 4
+# MB, 216 pairs 1.30 against 1.15, 6 MB, 328 pairs 1.04 against 1.14; head_dim 96
+# INT2, 8 MB, 3 chunks 0.80 against 0.73).  Reads of small windows on a stream
+# beside the decodes took longer than both (1.84 ms for the 24-token blocks).
+_COPY_VECTOR_PAIRS = 256
+_COPY_VECTOR_BYTES = 7 << 18
+_COPY_VECTOR_CHUNKS = 5
 # device bytes of packed arrays a direct decode fills at a time (1.2 ms of PCIe)
 _WINDOW_BYTES = 64 << 20
 
@@ -347,8 +358,9 @@ class RecordStager:
             t0 = time.perf_counter()
             reads = None
             try:
-                if self._direct(query, fill):
-                    acc, reads = self._loop_direct(query, sm_scale, fill.host, block_ids, status)
+                direct = self._direct(query, sm_scale, fill, len(block_ids))
+                if direct is not None:
+                    acc, reads = self._loop_direct(query, sm_scale, fill.host, block_ids, status, direct)
                 elif isinstance(self.backend, HipAttentionBackend) and query.dtype in _native.QUERY_DTYPES:
                     acc = self._loop_native(query, sm_scale, chunks, fill, status)
                 else:
@@ -424,11 +436,15 @@ class RecordStager:
             descs[n] = d
         return descs, need
 
-    def _direct(self, query: torch.Tensor, fill: Fill) -> bool:
-        """Whether the gather kernel reads the records from host memory itself:
-        chunks too small for copies at PCIe's rate, and a layout that the
-        gather reads once (all four arrays whole 16-byte chunks)."""
-        return (
+    def _direct(self, query: torch.Tensor, sm_scale: float, fill: Fill, total: int) -> int | None:
+        """The decode kernel of a run whose records the gather kernel reads from
+        host memory itself: that of one of its chunks (AUTO's choice for few
+        blocks; its output error is the smaller one, 16K tokens, 8 kv heads, fp32:
+        6.4e-5 against 9.1e-5 for a whole window's).  None where chunks are copied:
+        large enough for copies at PCIe's rate or for the vector kernel to run
+        behind them, or a layout that the gather would read twice (not all four
+        arrays whole 16-byte chunks)."""
+        if not (
             isinstance(fill, HostFill)
             and isinstance(self.backend, HipAttentionBackend)
             and query.dtype in _native.QUERY_DTYPES
@@ -436,14 +452,34 @@ class RecordStager:
             and self.layout.packed % 16 == 0
             and self.layout.scales % 16 == 0
             and fill.host.device_readable()
+        ):
+            return None
+        blocks = min(self.stage_blocks, total)
+        descs, _ = self._describe(query.contiguous(), sm_scale, {blocks})
+        L, b = self.layout, self.slots[0].batch.data_ptr()
+        kernel, tiled, splits = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_int(0)
+        rc = _native.load().kvssd_hip_decode_plan(
+            ctypes.byref(descs[blocks]), b + L.off_kp, b + L.off_vp, b + L.off_ks, b + L.off_vs,
+            ctypes.byref(kernel), ctypes.byref(tiled), ctypes.byref(splits),
         )
+        _native.check(rc, "kvssd_hip_decode_plan")
+        vector = kernel.value == _native.KERNEL_GENERAL and not tiled.value
+        if (
+            vector
+            and blocks * self.spec.kv_heads >= _COPY_VECTOR_PAIRS
+            and blocks * self.spec.record_bytes >= _COPY_VECTOR_BYTES
+            and total > (_COPY_VECTOR_CHUNKS - 1) * blocks
+        ):
+            return None
+        return kernel.value
 
-    def _loop_direct(self, query, sm_scale, host, block_ids, status):
+    def _loop_direct(self, query, sm_scale, host, block_ids, status, kernel):
         """Gather each window of the selection straight out of page-locked host
         memory and decode it in one call: on one stream and with no copies, two
-        launches a window (the gather, at PCIe's rate, takes ~100 times the
-        decode's time, so overlapping them would gain nothing).  Returns the
-        result and the host memory that the launches read."""
+        launches a window (the gather, at PCIe's rate, takes ~100 times the time
+        of a matrix-core decode, so overlapping them would gain nothing; for the
+        vector kernel see _COPY_VECTOR_PAIRS).  ``kernel`` takes the decodes.
+        Returns the result and the host memory that the launches read."""
         spec = self.spec
         lib = _native.load()
         q = query.contiguous()
@@ -452,14 +488,7 @@ class RecordStager:
         windows = -(-total // max(1, self.window_bytes // per_block))
         size = -(-total // windows)
         counts = [min(size, total - i) for i in range(0, total, size)]
-        # a window takes the kernel that a chunk of it would (AUTO's choice for few
-        # blocks): its output error is the smaller one (16K tokens, 8 kv heads, fp32:
-        # 6.4e-5 against 9.1e-5)
-        chunk, _ = self._describe(q, sm_scale, {min(self.stage_blocks, total)})
-        kernel = ctypes.c_int(0)
-        rc = lib.kvssd_hip_decode_kernel(ctypes.byref(next(iter(chunk.values()))), ctypes.byref(kernel))
-        _native.check(rc, "kvssd_hip_decode_kernel")
-        descs, need = self._describe(q, sm_scale, set(counts), kernel.value)
+        descs, need = self._describe(q, sm_scale, set(counts), kernel)
         L = BatchLayout.for_spec(spec, size)
         if self._window is None or self._window.numel() < L.total:
             self._window = torch.empty(L.total, dtype=torch.uint8, device=self.device)

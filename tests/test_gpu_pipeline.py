@@ -385,3 +385,37 @@ def test_ring_waits_for_its_memorys_earlier_uses(cuda_device):
     out, lse = stager.run(query, 0.1, 0, list(range(12)), lambda ids, slot: HostRecords(pinned, list(range(12))).spans(ids, spec.record_bytes))
     torch.testing.assert_close(out, ref_out, atol=1e-4, rtol=1e-3)
     torch.testing.assert_close(lse, ref_lse, atol=1e-4, rtol=1e-4)
+
+
+@pytest.mark.parametrize(("kv_heads", "head_dim", "group", "block_tokens", "chunk", "blocks", "direct"), [
+    # the matrix-core and the tiled kernel's layouts: read in place below 8 MiB a chunk
+    (8, 128, 32, 128, 4, 10, True), (8, 128, 32, 128, 55, 60, True), (8, 128, 32, 128, 56, 60, False), (8, 128, 32, 16, 160, 700, True),
+    # the vector kernel's: copied from 256 (block, head) pairs, 1.75 MiB and five chunks on
+    (8, 128, 32, 24, 60, 300, True), (8, 128, 32, 24, 70, 300, False), (8, 128, 32, 24, 70, 280, True),
+    (8, 192, 32, 128, 16, 70, True), (1, 192, 32, 16, 200, 900, True),
+])
+def test_host_resident_direct_or_copied(cuda_device, monkeypatch, kv_heads, head_dim, group, block_tokens, chunk, blocks, direct):
+    from kvssd import records_hip as R
+    from kvssd.format import CacheSpec
+    from kvssd.staging import HostRecords, RecordStager
+
+    dev = cuda_device
+    spec = CacheSpec(1, kv_heads, head_dim, block_tokens, 4, group)
+    gen = torch.Generator(device=dev).manual_seed(chunk)
+    kv = torch.randn(2, blocks * block_tokens - 5, kv_heads, head_dim, generator=gen, device=dev).half()
+    query = torch.randn(2 * kv_heads, head_dim, generator=gen, device=dev).half()
+    records, _ = R.encode_records(kv[0], kv[1], spec, 0)
+    pinned = torch.empty(records.shape, dtype=torch.uint8, pin_memory=True)
+    pinned.copy_(records)
+    backend = HipAttentionBackend()
+    stager = RecordStager(spec, dev, chunk, backend, torch.cuda.Stream(dev), torch.cuda.Stream(dev))
+    taken = []
+    for name in ("_loop_direct", "_loop_native"):
+        loop = getattr(stager, name)
+        monkeypatch.setattr(stager, name, lambda *a, _loop=loop, _name=name: taken.append(_name) or _loop(*a))
+    out, lse = stager.run(query, 0.2, 0, list(range(blocks)), stager.host_fill(HostRecords(pinned, list(range(blocks)))))
+    assert taken == ["_loop_direct" if direct else "_loop_native"]
+    pk, pv, sk, sv, valid, _ = R.gather_records(records.view(-1), spec, blocks)
+    ref_out, ref_lse = backend.run(query, PackedBatch(pk, pv, sk, sv, valid, 4, group), 0.2)
+    torch.testing.assert_close(out, ref_out, atol=1e-4, rtol=1e-3)
+    torch.testing.assert_close(lse, ref_lse, atol=1e-4, rtol=1e-4)
