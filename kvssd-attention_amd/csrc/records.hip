@@ -659,17 +659,26 @@ inline bool word_aligned(const void* src, const void* packed) {
   return (reinterpret_cast<uintptr_t>(src) & 15u) == 0 && (reinterpret_cast<uintptr_t>(packed) & 3u) == 0;
 }
 
+// threads of one launch, 2^34 INT4 values of the word form (a grid holds less than 2^32
+// of them, and of one of more only the rest runs, without an error)
+constexpr int64_t kMaxThreads = int64_t{1} << 31;
+
 template <typename T>
 void launch_quantize_t(const void* x, int64_t groups, int group_size, int bits, uint8_t* packed, uint16_t* scales,
                        hipStream_t s) {
   const int lanes = word_aligned(x, packed) ? word_lanes(group_size, bits) : 0;
-  const int64_t count = lanes > 0 ? groups * lanes : groups;
-  const dim3 grid(static_cast<unsigned>((count + 255) / 256));
-  const T* src = static_cast<const T*>(x);
-  if (bits == 4)
-    hipLaunchKernelGGL((quantize_kernel<T, 4>), grid, dim3(256), 0, s, src, count, group_size, lanes, packed, scales);
-  else
-    hipLaunchKernelGGL((quantize_kernel<T, 2>), grid, dim3(256), 0, s, src, count, group_size, lanes, packed, scales);
+  const int64_t most = lanes > 0 ? kMaxThreads / lanes : kMaxThreads;  // (lanes is a power of two)
+  for (int64_t g0 = 0; g0 < groups; g0 += most) {
+    const int64_t n = groups - g0 < most ? groups - g0 : most;
+    const int64_t count = lanes > 0 ? n * lanes : n;
+    const dim3 grid(static_cast<unsigned>((count + 255) / 256));
+    const T* src = static_cast<const T*>(x) + g0 * group_size;
+    uint8_t* codes = packed + g0 * (group_size * bits / 8);
+    if (bits == 4)
+      hipLaunchKernelGGL((quantize_kernel<T, 4>), grid, dim3(256), 0, s, src, count, group_size, lanes, codes, scales + g0);
+    else
+      hipLaunchKernelGGL((quantize_kernel<T, 2>), grid, dim3(256), 0, s, src, count, group_size, lanes, codes, scales + g0);
+  }
 }
 
 template <typename T, int PARTS>

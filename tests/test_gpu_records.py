@@ -420,3 +420,22 @@ def test_encode_wide_layers_few_records_keep_their_speed(cuda_device):
 
     small = fastest(CacheSpec(1, 24, 128, 64, 2, 32), torch.float32)
     assert fastest(CacheSpec(1, 24, 128, 128, 2, 32), torch.float32) < 1.4 * small
+
+
+def test_quantize_more_values_than_a_grid(cuda_device):
+    # 2^35 INT4 values are 2^32 words of codes, more threads than one launch takes: the rows at the
+    # ends and around the seams as in calls of their own
+    rows = (1 << 28) + 3
+    if torch.cuda.mem_get_info(cuda_device)[0] < 110 << 30:
+        pytest.skip("needs 82 GiB of device memory")
+    x = torch.empty(rows, 128, dtype=torch.float16, device=cuda_device)
+    gen = torch.Generator(device=cuda_device).manual_seed(9)
+    spots = [0, (1 << 27) - 2, (1 << 28) - 1]
+    for at in spots:
+        x[at : at + 4] = torch.randn(4, 128, generator=gen, device=cuda_device).half()
+    q = R.quantize(x, 4, 32)
+    for at in spots:
+        part = R.quantize(x[at : at + 4].clone(), 4, 32)
+        assert torch.equal(q.packed[at : at + 4], part.packed) and torch.equal(q.scales[at : at + 4], part.scales)
+    del x, q
+    torch.cuda.empty_cache()
