@@ -155,13 +155,11 @@ class HostRecords:
 
     def __post_init__(self) -> None:
         self.row_of = {b: i for i, b in enumerate(self.block_ids)}
-        self._device_readable: bool | None = None
 
     def device_readable(self) -> bool:
-        """Whether a kernel can read the records where they are (page-locked, rows back to back)."""
-        if self._device_readable is None:
-            self._device_readable = self.records.is_contiguous() and self.records.is_pinned()
-        return self._device_readable
+        """Whether a kernel can read the records where they are (page-locked, rows
+        back to back): asked of the tensor held now, each time (under 2 us)."""
+        return self.records.is_contiguous() and self.records.is_pinned()
 
     def spans(self, ids: Sequence[int], record_bytes: int) -> list[Span]:
         """One span per run of consecutive rows, in the order of ``ids``."""

@@ -419,3 +419,15 @@ def test_host_resident_direct_or_copied(cuda_device, monkeypatch, kv_heads, head
     ref_out, ref_lse = backend.run(query, PackedBatch(pk, pv, sk, sv, valid, 4, group), 0.2)
     torch.testing.assert_close(out, ref_out, atol=1e-4, rtol=1e-3)
     torch.testing.assert_close(lse, ref_lse, atol=1e-4, rtol=1e-4)
+
+
+def test_host_records_are_asked_each_time(cuda_device):
+    # records put in place of page-locked ones are not read by a kernel (nothing is launched here)
+    from kvssd.staging import HostRecords
+
+    host = HostRecords(torch.zeros(4, 4096, dtype=torch.uint8, pin_memory=True), [0, 1, 2, 3])
+    assert host.device_readable()
+    host.records = torch.zeros(4, 4096, dtype=torch.uint8)
+    assert not host.device_readable()
+    host.records = torch.zeros(4, 8192, dtype=torch.uint8, pin_memory=True)[:, :4096]
+    assert not host.device_readable()
