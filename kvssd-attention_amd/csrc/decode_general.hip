@@ -1,7 +1,7 @@
 // General fused decode kernel: every shape the reference accepts
 // (head_dim <= 256, any group size with head_dim % group_size == 0, INT2/INT4,
 // any GQA ratio, any block_tokens), fp32 arithmetic on the VALU.  It runs where
-// the tiled matrix-core kernel (decode_tile.hip, the same precision and 10-20
+// the tiled matrix-core kernel (decode_tile.hip, the same precision and 6 to 23
 // times its speed) does not apply: other head dims, more than 16 groups per
 // head, blocks that are no multiple of 16 tokens, unaligned arrays.
 //

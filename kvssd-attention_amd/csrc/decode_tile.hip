@@ -14,9 +14,11 @@
 // head_dim 256, groups of 64, bf16 222 -> 21.3 us; 16K tokens, head_dim 64 (the
 // kernel alone) 60 -> 10 us.  Output error against float64 (rms over 192 to 1,600
 // heads of a shape): INT4 0.53-0.89 times the vector kernel's, INT2 0.82-1.08.
-// What bounds it now: ~5 us of a workgroup's start and end (argument, table and
-// query round trips, the waves' merge), and in between its 64-byte pieces of
-// rows, which HBM serves at ~4 TB/s.
+// What bounds it now: a workgroup's start and end (argument, table and query
+// round trips, the waves' merge), and in between the VALU: of the 32K-token
+// decode above, 1,180 instructions a wave and 4 waves a SIMD, 7.9 us of issue
+// (the matrix cores are busy for 1.3 us); 1M tokens in 32-token blocks, 128
+// passes a SIMD, come in at 3.7 TB/s.
 //
 // Work split.  A workgroup of 4 waves owns one kv head, up to 16 / Gp of its
 // query heads (Gp: groups per head, rounded up to a power of two) and one
@@ -52,8 +54,9 @@ constexpr int kTileThreads = kWave * kTileWaves;
 constexpr int kChunkTok = 64;               // token slots of a wave's pass
 constexpr int kWRowBytes = 2 * kChunkTok + 16;  // one W row: 64 fp16 slots and a pad
 
-// Kernel arguments beyond the preloaded ones (query, pk, pv, sk, sv and the
-// four dwords: what the first loads of a decode without a table need).
+// Kernel arguments beyond the preloaded ones (query, pk, pv, sk, sv and four
+// dwords).  The first pass's addresses wait for a fetch of these: the block
+// table and the constants that find block ends are among them.
 struct TileTail {
   const int32_t* table;
   const int32_t* valid;
@@ -76,6 +79,8 @@ inline uint32_t pack_shape(int kv_heads, int groups, int group_shift, bool has_t
 
 // workgroups resident on a CU (4 waves each, one per SIMD), by registers and,
 // for head_dim 256, by LDS: what the register budget and the split plan count on
+// (of INT2, one-part, head_dim 256 with four or more groups, 158 registers and
+// 43 KB, three would fit)
 constexpr int tile_workgroups_per_cu(int head_dim, int hs, int parts) {
   return parts == 1 && (head_dim == 64 || (head_dim == 128 && hs == 1)) ? 4 : head_dim <= 128 ? 3 : 2;
 }

@@ -110,7 +110,9 @@ class HipAttentionBackend:
         )
 
     def kernel_for(self, query: torch.Tensor, batch: PackedBatch, sm_scale: float = 1.0) -> str:
-        """Name of the kernel ``run`` would launch for this shape ("general", "mfma" or "staged")."""
+        """Name of the kernel ``run`` would launch for this shape ("general", "mfma" or
+        "staged"; "general" stands for the tiled matrix-core kernel and, for the shapes
+        and alignments that it does not take, the vector kernel)."""
         desc = self.describe(query, batch, sm_scale)
         out = ctypes.c_int(0)
         _native.check(_native.load().kvssd_hip_decode_kernel(ctypes.byref(desc), ctypes.byref(out)), "decode_kernel")

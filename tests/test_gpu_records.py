@@ -101,7 +101,7 @@ SPECS = [
     CacheSpec(layers=1, kv_heads=1, head_dim=4, block_tokens=3, bits=2, group_size=4),
     # 55,296-byte payload: 4 rows of 16-byte chunks behind 10,240 virtual zero bytes
     CacheSpec(layers=1, kv_heads=8, head_dim=128, block_tokens=48, bits=4, group_size=32),
-    # 294,912-byte payload: beyond the chunked form's 256 KiB, general form
+    # 294,912-byte payload: 18 rows of 16-byte chunks, five groups of four rows
     CacheSpec(layers=1, kv_heads=8, head_dim=128, block_tokens=256, bits=4, group_size=32),
 ]
 
@@ -215,7 +215,7 @@ def test_gather_records_unaligned_outputs(cuda_device):
 @pytest.mark.parametrize("bits", [2, 4])
 def test_quantize_unaligned_source_matches(cuda_device, bits):
     # a source that is not 16-byte aligned takes the element-wise form; the
-    # register form (aligned, group 32) gives the same bytes
+    # word form (aligned) gives the same bytes
     gen = torch.Generator().manual_seed(21)
     x = torch.randn(301, 128, generator=gen).half()
     buf = torch.empty(301 * 128 + 1, dtype=torch.float16, device=cuda_device)
@@ -285,7 +285,7 @@ def test_quantize_around_ties(cuda_device, bits, dtype):
 def test_quantize_nan_and_infinity(cuda_device, bits, dtype):
     # a NaN takes code 0 and leaves its group's scale alone; a group with an infinity has an
     # infinite scale, so finite values take the middle code and the infinity (inf / inf) code 0;
-    # the register form (group 32) as the element-wise one (the same values in a shifted source)
+    # the word form as the element-wise one (the same values in a shifted source)
     gen = torch.Generator().manual_seed(17)
     x = torch.randn(64, 128, generator=gen)
     x[3, 5] = x[9, 64] = x[9, 71] = float("nan")
