@@ -419,7 +419,7 @@ def test_encode_wide_layers_few_records_keep_their_speed(cuda_device):
         return min(times)
 
     small = fastest(CacheSpec(1, 24, 128, 64, 2, 32), torch.float32)
-    assert fastest(CacheSpec(1, 24, 128, 128, 2, 32), torch.float32) < 1.4 * small
+    assert fastest(CacheSpec(1, 24, 128, 128, 2, 32), torch.float32) < 1.7 * small
 
 
 def test_quantize_more_values_than_a_grid(cuda_device):
